@@ -27,7 +27,7 @@ __device__ __forceinline__ void dma16(uint32_t lds, const void* gbase, uint32_t 
 }
 
 // dma16 into LDS lds + OFF: M0 is set from the scalar base plus the constant in one SALU
-// instruction (a kernel's ring position is a compile-time constant).
+// instruction (a kernel's ring position is a compile-time constant), which writes SCC.
 template <int OFF>
 __device__ __forceinline__ void dma16_at(uint32_t lds, const void* gbase, uint32_t voff) {
     if constexpr (OFF == 0)
@@ -36,7 +36,7 @@ __device__ __forceinline__ void dma16_at(uint32_t lds, const void* gbase, uint32
         asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                      :
                      : "s"(lds), "v"(voff), "s"(gbase), "n"(OFF)
-                     : "memory");
+                     : "memory", "scc");
 }
 
 // 12 bytes per lane global -> LDS: lane l's bytes go to LDS m0 + OFF + 16*l (the instruction keeps a
@@ -52,7 +52,7 @@ __device__ __forceinline__ void dma12_at(uint32_t lds, const void* gbase, uint32
         asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx3 %1, %2"
                      :
                      : "s"(lds), "v"(voff), "s"(gbase), "n"(OFF)
-                     : "memory");
+                     : "memory", "scc");
 }
 
 // Same with a per-lane 64-bit global address.
