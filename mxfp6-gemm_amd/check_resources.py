@@ -55,7 +55,7 @@ def violations(kernels):
 
 
 def family(name):
-    for fam in ("wide_kernel", "slab_kernel", "direct_kernel", "reduce_splitk_kernel",
+    for fam in ("wide_kernel", "stream_kernel", "slab_kernel", "direct_kernel", "reduce_splitk_kernel",
                 "repack_rows_kernel", "prep"):
         if fam in name:
             return fam

@@ -49,6 +49,7 @@
 #include "lds_dma.hpp"
 #include "repack_kernel.hpp"
 #include "slab_run.hpp"
+#include "stream_kernel.hpp"
 #include "wide_kernel.hpp"
 
 namespace mxfp6_dev {
@@ -356,9 +357,9 @@ hipError_t slab_kernel_launch(const mxfp6_launch_desc* d, const uint8_t* A, hipS
 }
 
 // Ring depth per tile: as many slabs as fit 160 KiB of LDS (128 x 128 and 32 x 128: half of it,
-// two workgroups per CU). MASK when the tile does not divide M x N. Returns 0, or 2 when a launch
-// fails.
-template <int MT, int NT, int WM, int WN, int XG, int NS, typename KT, bool SPLIT>
+// two workgroups per CU). MASK when the tile does not divide M x N. ROWS: row-major A is
+// read by this kernel (false: d's A is repacked or preshuffled). Returns 0, or 2 when a launch fails.
+template <int MT, int NT, int WM, int WN, int XG, int NS, typename KT, bool SPLIT, bool ROWS = true>
 int slab_launch_t(const mxfp6_launch_desc* d, hipStream_t st) {
     static_assert(SlabGeom<MT, NT, WM, WN, NS>::LDS <= 160 * 1024, "LDS budget");
     if (d->a_layout == MXFP6_A_ROWS_SWIZZLED) return 2;  // a staging of the wide tiles only
@@ -372,11 +373,11 @@ int slab_launch_t(const mxfp6_launch_desc* d, hipStream_t st) {
         A = static_cast<const uint8_t*>(d->Ash);
     }
     hipError_t e;
-    if (d->a_layout == MXFP6_A_ROWS) {
+    if (ROWS && d->a_layout == MXFP6_A_ROWS) {
         if (mask)
-            e = slab_kernel_launch<MT, NT, WM, WN, XG, NS, KT, SPLIT, false, true>(d, A, st);
+            e = slab_kernel_launch<MT, NT, WM, WN, XG, NS, KT, SPLIT, !ROWS, true>(d, A, st);
         else
-            e = slab_kernel_launch<MT, NT, WM, WN, XG, NS, KT, SPLIT, false, false>(d, A, st);
+            e = slab_kernel_launch<MT, NT, WM, WN, XG, NS, KT, SPLIT, !ROWS, false>(d, A, st);
     } else {
         if (mask)
             e = slab_kernel_launch<MT, NT, WM, WN, XG, NS, KT, SPLIT, true, true>(d, A, st);
@@ -384,6 +385,14 @@ int slab_launch_t(const mxfp6_launch_desc* d, hipStream_t st) {
             e = slab_kernel_launch<MT, NT, WM, WN, XG, NS, KT, SPLIT, true, false>(d, A, st);
     }
     return e == hipSuccess ? 0 : 2;
+}
+
+// The skinny tiles: row-major A on the stream kernel, A repacked or preshuffled on the slab kernel
+// with one wave row and four wave columns.
+template <int MT, int NT, typename KT, bool SPLIT>
+int skinny_launch(const mxfp6_launch_desc* d, hipStream_t st) {
+    if (d->a_layout == MXFP6_A_ROWS) return stream_launch<MT / 32, NT / 128, KT, SPLIT>(d, st);
+    return slab_launch_t<MT, NT, 1, 4, 4, 8, KT, SPLIT, false>(d, st);
 }
 
 // The wide tiles (four waves side by side, B straight to registers): the A repack first when
@@ -437,11 +446,11 @@ int slab_run(const mxfp6_launch_desc* d, hipStream_t st) {
     if (d->MT == 128 && d->NT == 256 && d->mpw == 4) return wide_launch_t<4, 2, 8, KT, SPLIT>(d, st);
     if (d->MT == 256 && d->NT == 256 && d->npw == 2) return wide_launch_t<8, 2, 4, KT, SPLIT>(d, st);
     if (d->MT == 128 && d->NT == 384) return wide_launch_t<4, 3, 8, KT, SPLIT>(d, st);
-    // skinny tiles: one wave row, four wave columns, a deeper ring
-    if (d->MT == 32 && d->NT == 128) return slab_launch_t<32, 128, 1, 4, 4, 8, KT, SPLIT>(d, st);
-    if (d->MT == 32 && d->NT == 256) return slab_launch_t<32, 256, 1, 4, 4, 8, KT, SPLIT>(d, st);
-    if (d->MT == 64 && d->NT == 128) return slab_launch_t<64, 128, 1, 4, 4, 8, KT, SPLIT>(d, st);
-    if (d->MT == 64 && d->NT == 256) return slab_launch_t<64, 256, 1, 4, 4, 8, KT, SPLIT>(d, st);
+    // skinny tiles: the stream kernel on row-major A, here preshuffled A (a deeper ring)
+    if (d->MT == 32 && d->NT == 128) return skinny_launch<32, 128, KT, SPLIT>(d, st);
+    if (d->MT == 32 && d->NT == 256) return skinny_launch<32, 256, KT, SPLIT>(d, st);
+    if (d->MT == 64 && d->NT == 128) return skinny_launch<64, 128, KT, SPLIT>(d, st);
+    if (d->MT == 64 && d->NT == 256) return skinny_launch<64, 256, KT, SPLIT>(d, st);
     if (d->MT == 128 && d->NT == 128) return slab_launch_t<128, 128, 2, 2, 4, 6, KT, SPLIT>(d, st);
     if (d->MT == 128 && d->NT == 256) return slab_launch_t<128, 256, 2, 2, 4, 8, KT, SPLIT>(d, st);
     if (d->MT == 256 && d->NT == 192) return slab_launch_t<256, 192, 2, 2, 4, 6, KT, SPLIT>(d, st);

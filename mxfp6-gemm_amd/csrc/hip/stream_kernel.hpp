@@ -1,0 +1,329 @@
+// Stream kernels of libmxfp6gemm for gfx950: the skinny tiles (32 and 64 rows) on row-major A, B read
+// once and straight into registers.
+//
+// A workgroup computes an MT x NT tile of D with MT = 32 MB and NT = 32 NPW WN: WN computing waves
+// side by side, each owning all MT rows and 32 NPW columns, and one copying wave. (MB, NPW) is the
+// tile's scale grouping: 32 x 128 (1, 1), 32 x 256 (1, 2), 64 x 128 (2, 1), 64 x 256 (2, 2); WN does
+// not change the arithmetic of a wave, so the output bits are the tile's for every WN.
+//   B       each computing wave loads its own blocks from the preshuffled layout into MFMA operand
+//           registers, L = 2 K-tiles ahead (per 64-wide slab and block a 16- and an 8-byte load a
+//           lane, contiguous), and its scales with them; a slab's loads for K-tile c + L are issued
+//           right after the MFMAs that read K-tile c's.
+//   A       chunks of CK = 2 K-tiles, copied by the copying wave along the rows (a row's 288 bytes
+//           are 3.1 cache lines on average, where two K-tile pieces of 144 bytes take 4) into a
+//           ring of NB = 3 LDS buffers, rows 304 bytes apart (16-byte pieces, one of padding), with
+//           the A scales of the chunk (one 12-byte copy a K-tile). A computing wave reads K-tile
+//           c + 1 from LDS into the other of two register sets while it multiplies K-tile c.
+//   sync    one workgroup barrier per chunk: the copying wave has waited for chunk g + 1 (its own
+//           vmcnt count: it issues nothing else), every computing wave for its reads of chunk g,
+//           whose buffer then takes chunk g + NB.
+// What bounds it: a CU keeps only about 32 KB of cache misses in flight (its L1's lines), whether
+// they go to registers or to LDS: 64 x 8192 x 8192 on 64 CUs moved 29 KB/us a CU from HBM and 48 from
+// the Infinity Cache, the same with 2, 4 or 6 K-tiles of loads ahead. So lead past two K-tiles is
+// worth nothing; the lines of A, the padded scale dwords and the number of CUs in use are what
+// counts. That is why A comes in two K-tiles per row piece, only one wave loads A's scales, and WN
+// shrinks when the grid is small (stream_launch). 64 x 28672 x 8192 (three operand sets in turn,
+// B from HBM): 52.1 us on the slab kernel (B and A through LDS a slab at a time, every wave
+// copying), 38.2 here: 5.0 TB/s of operands; without A's copies and scales 30.5.
+// NT: B's loads are nontemporal where B exceeds half the last-level cache and is read by one tile
+// row: 44.8 -> 39.1 us at 64 x 28672 x 8192 (B 176 MB), while B that would have stayed in the cache
+// loses (64 x 8192 x 8192, B 50 MB: 20.9 -> 31.4 us).
+// MASK (ragged M or N): rows past M repeat the last one, blocks and scale groups past the end the last
+// that exists; stores are masked.
+#pragma once
+
+#include "../hip_layer.h"
+#include "device_common.hpp"
+#include "epilogue.hpp"
+#include "lds_dma.hpp"
+#include "wide_kernel.hpp"
+
+namespace mxfp6_dev {
+
+template <int MB_, int NPW_, int WN_>
+struct StreamGeom {
+    static constexpr int MB = MB_, NPW = NPW_, WN = WN_;
+    static constexpr int L = 2;                                 // K-tiles of B in flight
+    static constexpr int CK = 2;                                // K-tiles of A a chunk
+    static constexpr int NB = 3;                                // chunk buffers
+    static constexpr int MT = 32 * MB, NT = 32 * NPW * WN;
+    static constexpr int THREADS = 64 * (WN + 1);
+    static constexpr int ROW = 9 * CK + 1;                      // 16-byte LDS pieces a row, one of padding
+    static constexpr int PIECES = MT * ROW;
+    static constexpr int COPIES = (PIECES + 63) / 64;           // wave copies of a chunk's rows
+    static constexpr int OPS = COPIES + CK;                     // and one of each K-tile's scales
+    static constexpr int CST = OPS * 1024;                      // LDS buffer stride
+    static constexpr int LDS = NB * CST;
+    static constexpr int PASS = 2;                              // K-tiles of a pass of the K loop
+    static_assert(PASS % CK == 0 && PASS % L == 0 && PASS % 2 == 0, "ring positions are constants");
+    static_assert((NB - 1) * OPS <= 63, "vmcnt range");
+    static_assert(LDS <= 160 * 1024, "LDS budget");
+};
+
+// f(T), f(T + 1), ... for the first `left` of the PASS positions (left < PASS).
+template <int T, int PASS, typename F>
+__device__ __forceinline__ void stream_tail(int left, F&& f) {
+    if constexpr (T + 1 < PASS) {
+        if (left > 0) {
+            f(std::integral_constant<int, T>{});
+            stream_tail<T + 1, PASS>(left - 1, f);
+        }
+    }
+}
+
+template <int MB_, int NPW_, int WN_, int XG, typename OutT, bool SPLIT, bool MASK, bool NTB>
+__global__ void __launch_bounds__(64 * (WN_ + 1), 1)
+    stream_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ Bsh,
+                  const uint8_t* __restrict__ sA, const uint8_t* __restrict__ sB,
+                  OutT* __restrict__ D, float* __restrict__ ws, int M, int N, int Kp,
+                  int A_row_bytes, int S) {
+    using G = StreamGeom<MB_, NPW_, WN_>;
+    constexpr int MT = G::MT, NT = G::NT, MB = G::MB, NPW = G::NPW, WN = G::WN, L = G::L;
+    constexpr int CK = G::CK, NB = G::NB;
+    constexpr int AUX = NTB ? 2 : 0;  // cache policy of the B loads (2: nontemporal)
+    __shared__ __attribute__((aligned(1024))) char lds[G::LDS];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int wg_m = blockIdx.x, wg_n = blockIdx.y, wg_z = SPLIT ? (int)blockIdx.z : 0;
+    if constexpr (XG > 0) {
+        const int gm = (int)gridDim.x, gn = (int)gridDim.y;
+        if (!SPLIT || (gm * gn) % NXCD == 0)
+            xcd_tile(gm, gn, XG, (int)(blockIdx.y * gridDim.x + blockIdx.x), wg_m, wg_n);
+    }
+    const int k64n = Kp / 64, k_tiles = Kp / 192;
+    int kt0 = 0, nkt = k_tiles;
+    if (SPLIT) split_segment(k_tiles, S, wg_z, kt0, nkt);
+    const int kt_last = kt0 + nkt - 1;
+
+    if (wave == WN) {
+        // the copying wave: copy i moves LDS piece p = 64 i + l of a chunk (16 bytes, lane l) from
+        // piece p % ROW of row p / ROW; the padding piece is not copied, nor are the pieces past the
+        // segment's end. Every copy has at least one lane to copy, so a chunk is OPS operations.
+        const int rows = MASK ? min(MT, M - wg_m * MT) : MT;
+        const uint8_t* a_tile = A + (size_t)wg_m * MT * A_row_bytes + (size_t)kt0 * (SUBS * SLAB_BYTES);
+        uint32_t voff[G::COPIES];
+#pragma unroll
+        for (int i = 0; i < G::COPIES; i++) {
+            const int p = i * 64 + lane, row = p / G::ROW, col = p - row * G::ROW;
+            voff[i] = p < G::PIECES && col < 9 * CK
+                          ? (uint32_t)((MASK ? min(row, rows - 1) : row) * A_row_bytes + 16 * col)
+                          : ~0u;
+        }
+        int ga = wg_m;
+        if (MASK) ga = min(ga, ((M + 31) / 32 + MB - 1) / MB - 1);
+        const uint8_t* sa_grp = sA + ((size_t)ga * k_tiles + kt0) * 64 * 12;
+        const uint32_t lds0 = lds_u32(lds), sc_voff = 12 * lane;
+        const int nch = (nkt + CK - 1) / CK;
+        auto copy = [&](int ch) {
+            const uint8_t* src = a_tile + (size_t)ch * (CK * SUBS * SLAB_BYTES);
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + ch % NB * G::CST);
+            const int kts = min(CK, nkt - ch * CK);
+            if (kts == CK) {
+#pragma unroll
+                for (int i = 0; i < G::COPIES; i++)
+                    if (voff[i] != ~0u) dma16(dst + i * 1024, src, voff[i]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < G::COPIES; i++) {
+                    const int col = (i * 64 + lane) % G::ROW;
+                    if (voff[i] != ~0u && col < 9 * kts) dma16(dst + i * 1024, src, voff[i]);
+                }
+            }
+            const uint32_t sdst = __builtin_amdgcn_readfirstlane(dst + G::COPIES * 1024);
+            for (int t = 0; t < CK; t++)
+                dma12_at<0>(sdst + t * 1024, sa_grp + (size_t)(ch * CK + min(t, kts - 1)) * 768, sc_voff);
+        };
+        for (int ch = 0; ch < NB && ch < nch; ch++) copy(ch);
+        // chunk ch landed, up to NB - 1 newer ones (OPS copies each) in flight
+        auto landed = [&](int ch, auto newer) {
+            if (ch + decltype(newer)::value < nch)
+                wait_vmcnt<decltype(newer)::value * G::OPS>();
+            else
+                wait_vmcnt0();
+        };
+        landed(0, std::integral_constant<int, NB - 1>{});
+        ring_barrier();
+        for (int ch = 0; ch < nkt / CK; ch++) {
+            landed(ch + 1, std::integral_constant<int, NB - 2>{});
+            ring_barrier();  // chunk ch + 1 landed, chunk ch read by every wave
+            if (ch + NB < nch) copy(ch + NB);
+        }
+        return;
+    }
+
+    const int b_blk_last = (N + 31) / 32 - 1;
+    rsrc_t b_rs[NPW];
+#pragma unroll
+    for (int ni = 0; ni < NPW; ni++) {
+        int blk = wg_n * (NT / 32) + wave * NPW + ni;
+        if (MASK) blk = min(blk, b_blk_last);
+        b_rs[ni] = raw_rsrc(opaque_gptr(Bsh + (size_t)blk * k64n * OPBLK_BYTES));
+    }
+    int gb = wg_n * WN + wave;
+    if (MASK) gb = min(gb, ((N + 31) / 32 + NPW - 1) / NPW - 1);
+    const rsrc_t sb_rs = raw_rsrc(opaque_gptr(sB + (size_t)gb * k_tiles * 64 * 12));
+    const int v_b0 = (int)opaque_v(16 * lane), v_b1 = (int)opaque_v(1024 + 8 * lane);
+    const int v_sc = (int)opaque_v(12 * lane);
+
+    v8i RB[L][SUBS][NPW];  // B operands and scales of K-tile c in slot c % L
+    v3i sc_b[L];
+    auto load_b = [&](v8i& v, int ni, int kt, int s) {
+        const int so = kt * (SUBS * OPBLK_BYTES);
+        const v4i y0 = __builtin_bit_cast(
+            v4i, __builtin_amdgcn_raw_buffer_load_b128(b_rs[ni], v_b0 + s * OPBLK_BYTES, so, AUX));
+        const v2i y1 = __builtin_bit_cast(
+            v2i, __builtin_amdgcn_raw_buffer_load_b64(b_rs[ni], v_b1 + s * OPBLK_BYTES, so, AUX));
+        const v4i y1w = __builtin_shufflevector(y1, y1, 0, 1, -1, -1);
+        v = __builtin_shufflevector(y0, y1w, 0, 1, 2, 3, 4, 5, -1, -1);
+    };
+    auto load_scales = [&](v3i& b, int kt) {
+        b = __builtin_bit_cast(v3i, __builtin_amdgcn_raw_buffer_load_b96(sb_rs, v_sc, kt * 768, AUX));
+    };
+    const lds_cptr lds3 = (lds_cptr)lds;
+    const uint32_t a_rd = (uint32_t)((lane & 31) * G::ROW * 16 + (lane >> 5) * 24);
+
+    v16f acc[MB][NPW];
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+        for (int j = 0; j < NPW; j++) acc[i][j] = v16f{};
+
+#pragma unroll
+    for (int c = 0; c < L; c++) {
+        const int kt = min(kt0 + c, kt_last);
+#pragma unroll
+        for (int s = 0; s < SUBS; s++)
+#pragma unroll
+            for (int ni = 0; ni < NPW; ni++) {
+                load_b(RB[c][s][ni], ni, kt, s);
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        load_scales(sc_b[c], kt);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // A operands and scales of a K-tile, two sets
+    v8i RA[2][SUBS][MB];
+    v3i sc_a[2];
+    auto read_a = [&](auto qq, auto tt, int buf) {
+        constexpr int Q = decltype(qq)::value, KT = decltype(tt)::value;
+        const uint32_t base = opaque_v(a_rd + buf * G::CST);
+        sc_a[Q] = *reinterpret_cast<const __attribute__((address_space(3))) v3i*>(
+            lds3 + opaque_v(16 * lane + buf * G::CST) + (G::COPIES + KT) * 1024);
+#pragma unroll
+        for (int s = 0; s < SUBS; s++)
+#pragma unroll
+            for (int mi = 0; mi < MB; mi++) {
+                const v6i_a8 x = *reinterpret_cast<const __attribute__((address_space(3))) v6i_a8*>(
+                    lds3 + base + mi * 32 * G::ROW * 16 + KT * SUBS * SLAB_BYTES + s * SLAB_BYTES);
+                RA[Q][s][mi] = __builtin_shufflevector(x, x, 0, 1, 2, 3, 4, 5, -1, -1);
+            }
+    };
+    ring_barrier();
+    read_a(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, 0);
+    int buf = 0;
+    auto ktile = [&](int c, auto tt) {
+        constexpr int T = decltype(tt)::value % L, Q = decltype(tt)::value % 2;
+        constexpr int NEXT = (decltype(tt)::value + 1) % CK;
+        if constexpr (NEXT == 0) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            ring_barrier();
+            buf = buf == NB - 1 ? 0 : buf + 1;
+        }
+        read_a(std::integral_constant<int, 1 - Q>{}, std::integral_constant<int, NEXT>{}, buf);
+        __builtin_amdgcn_sched_barrier(0);
+        const int kt_next = min(kt0 + c + L, kt_last);
+        const v3i ca = sc_a[Q], cb = sc_b[T];
+#pragma unroll
+        for (int s = 0; s < SUBS; s++) {
+            const int sa = s == 0 ? ca.x : s == 1 ? ca.y : ca.z;
+            const int sb = s == 0 ? cb.x : s == 1 ? cb.y : cb.z;
+#pragma unroll
+            for (int ni = 0; ni < NPW; ni++) {
+#pragma unroll
+                for (int mi = 0; mi < MB; mi++)
+                    wide_mfma<MB, NPW>(acc, mi, ni, RA[Q][s][mi], RB[T][s][ni], sa, sb);
+                __builtin_amdgcn_sched_barrier(0);
+                load_b(RB[T][s][ni], ni, kt_next, s);
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+                if (s == SUBS - 1 && ni == NPW - 1) {
+                    load_scales(sc_b[T], kt_next);
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+    };
+    // Whole passes, then the K-tiles left. No exit inside a pass: where it met the loop's back edge
+    // the compiler would wait for loads just issued. For the same reason a K-tile's scale load comes
+    // after the last MFMA that uses the slot's old ones (a copy of them would be waited for).
+    constexpr int PASS = G::PASS;
+    int c = 0;
+    for (; c + PASS <= nkt; c += PASS) static_for<PASS>([&](auto tt) { ktile(c + decltype(tt)::value, tt); });
+    stream_tail<0, PASS>(nkt - c, [&](auto tt) { ktile(c + decltype(tt)::value, tt); });
+    const int le = lane_id();
+    store_tile<MB, NPW, OutT, SPLIT, MASK>(acc, D, ws, M, N, wg_m * MT + 4 * (le >> 5),
+                                           wg_n * NT + wave * NPW * 32 + (le & 31), le, wg_z);
+}
+
+// One launch for a tile of grouping (MB, NPW), four computing waves wide as the router counts it.
+// The K-segment partials go to d->ws when SPLIT. Fewer computing waves a workgroup where four
+// would leave CUs idle or load them unevenly (three operand sets in turn, 177 shapes with up to
+// 4,500 workgroups; the slab kernel was 1.02-1.63x slower on every one of them):
+//   one 32-column block a wave (NPW 1): two waves below 3/5 of the CUs, and on 32 rows one
+//   where two stay below that as well (32 x 384 x 12928 in 16 segments, 48 workgroups of four:
+//   four 1.13x, two 1.04x, one 1; 16 x 1024 x 10880, 128: four 1.11x, two 1);
+//   two blocks a wave: two waves on more workgroups than CUs, which four waves' registers run
+//   one round at a time (96 x 23552 x 2112, 276 workgroups: four 1.25x two; 2240 x 2176 x 576,
+//   315: 1.21x; on 144-256 workgroups four are 0-12% faster).
+template <int MB, int NPW, int WN, typename KT, bool SPLIT>
+hipError_t stream_launch_w(const mxfp6_launch_desc* d, bool ntb, hipStream_t st) {
+    using G = StreamGeom<MB, NPW, WN>;
+    const bool mask = d->M % G::MT != 0 || d->N % G::NT != 0;
+    const dim3 grid((unsigned)((d->M + G::MT - 1) / G::MT), (unsigned)((d->N + G::NT - 1) / G::NT),
+                    (unsigned)d->splits);
+    auto k = mask ? stream_kernel<MB, NPW, WN, 4, KT, SPLIT, true, false>
+                  : stream_kernel<MB, NPW, WN, 4, KT, SPLIT, false, false>;
+    if constexpr (WN == 4) {
+        if (ntb)
+            k = mask ? stream_kernel<MB, NPW, WN, 4, KT, SPLIT, true, true>
+                     : stream_kernel<MB, NPW, WN, 4, KT, SPLIT, false, true>;
+    }
+    return launch_kernel(k, grid, dim3(G::THREADS), st, static_cast<const uint8_t*>(d->A),
+                         static_cast<const uint8_t*>(d->Bsh), d->sA, d->sB,
+                         SPLIT ? nullptr : static_cast<KT*>(d->D), SPLIT ? d->ws : nullptr, d->M,
+                         d->N, d->Kp, d->A_row_bytes, SPLIT ? d->splits : 1);
+}
+
+// Returns 0, or 2 when the launch fails.
+template <int MB, int NPW, typename KT, bool SPLIT>
+int stream_launch(const mxfp6_launch_desc* d, hipStream_t st) {
+    const int reported = mxfp6_hip_device_cus();
+    const long cus = reported > 0 ? reported : 256;
+    auto wgs = [&](int wn) {
+        return (long)((d->M + 32 * MB - 1) / (32 * MB)) * ((d->N + 32 * NPW * wn - 1) / (32 * NPW * wn)) *
+               d->splits;
+    };
+    // B read once (one tile row) and more than half of the 256 MiB last-level cache
+    const bool ntb = d->M <= 32 * MB && (double)d->N * (d->Kp / 4 * 3) > 128.0 * (1 << 20);
+    hipError_t e;
+    if constexpr (NPW == 1) {
+        if (MB == 1 && 5 * wgs(2) < 3 * cus)
+            e = stream_launch_w<MB, NPW, MB == 1 ? 1 : 2, KT, SPLIT>(d, ntb, st);
+        else if (5 * wgs(4) < 3 * cus)
+            e = stream_launch_w<MB, NPW, 2, KT, SPLIT>(d, ntb, st);
+        else
+            e = stream_launch_w<MB, NPW, 4, KT, SPLIT>(d, ntb, st);
+    } else {
+        if (wgs(4) > cus && !ntb)
+            e = stream_launch_w<MB, NPW, 2, KT, SPLIT>(d, ntb, st);
+        else
+            e = stream_launch_w<MB, NPW, 4, KT, SPLIT>(d, ntb, st);
+    }
+    return e == hipSuccess ? 0 : 2;
+}
+
+}  // namespace mxfp6_dev
