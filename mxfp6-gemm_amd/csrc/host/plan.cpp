@@ -410,7 +410,9 @@ bool streams_output(int out_type, int M, int N, int Kp, const TileChoice& tc, in
     const double in = (double)M * A_row_bytes + (repack ? ((M + 31) / 32 * 32) * packed : 0.0) +
                       (double)N * packed + (double)(M + N) * (Kp / 32);
     const double out = (double)M * N * (out_type == 0 ? 4 : 2);  // FP32 or a 16-bit type
-    return in <= LLC_BYTES && in + out > STREAM_FOOTPRINT_BYTES;
+    if (in > LLC_BYTES) return false;
+    return in + out > STREAM_FOOTPRINT_BYTES ||
+           (in + out > LLC_BYTES / 2 && out >= STREAM_D_RATIO * in);
 }
 
 // ws: the workspace of the plan (S, a_layout): split partials first, then (MXFP6_A_REPACK) the

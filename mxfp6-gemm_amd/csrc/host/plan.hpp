@@ -34,8 +34,18 @@ constexpr double PLAN_MIN_GAIN = 0.01;     // lead a more complex plan needs ove
 // 16384x16384x4096, 1024x102272x2048, 2048x102272x1024), plain stores 5-12% faster below it
 // (8192x8192x2048, 8192x12288x2048, 2048x51200x1024), no difference once the operands alone
 // exceed the cache (2048x102272x4096).
+// Below that footprint, from half the cache on, it does so where D is at least
+// STREAM_D_RATIO times what it reads (short K, many tile rows). Two such calls in a row, on operands
+// and outputs of their own as a program's layers are, then no longer fit the cache together, and the
+// plain stores of one wait for the other's to be written back. Three sets in turn, plain -> streamed:
+// 8192x8192x1024 (D 10x the operands) 100.7 -> 82.4 us, 16384x8192x512 155.8 -> 117.5,
+// 4096x16384x768 79.3 -> 68.0, 16384x4096x512 76.7 -> 72.9; the same set over and over 83.0 -> 84.6,
+// 130.6 -> 116.1, 78.8 -> 67.3, 97.6 -> 65.0. Below half the cache no gain (8192x7168x1024 81.6 ->
+// 80.3, 8192x6144x1024 61.5 -> 68.5), nor at lower ratios where the operands weigh more
+// (2048x28672x1024, 4x: 81.9 -> 85.7; the same set 8192x8192x2048, 5x: 111.0 -> 115.1).
 constexpr double LLC_BYTES = 268435456.0;
 constexpr double STREAM_FOOTPRINT_BYTES = 280e6;
+constexpr double STREAM_D_RATIO = 8.0;
 
 TileChoice route(int M, int N, int Kp);
 int splitk_segments(int M, int N, int Kp);

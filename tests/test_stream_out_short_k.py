@@ -1,0 +1,32 @@
+"""Unsplit plans on wide tiles whose operands and D fill half the 256 MiB last-level cache or more with
+a D of at least 8 times the operands (short K) write D with nontemporal stores: the rule's edges, and
+the values against the direct kernel bit for bit."""
+import pytest
+
+import checks
+import mxfp6_amd as mx
+
+
+@pytest.mark.parametrize("M,N,K,out_type,want", [
+    (8192, 8192, 1024, mx.OUT_BF16, True),    # D 134 MB, 10x the operands
+    (8192, 7936, 960, mx.OUT_BF16, True),     # 130 + 12 MB: over half the cache
+    (8192, 7168, 1024, mx.OUT_BF16, False),   # 131 MB in all: under it
+    (8192, 8192, 1536, mx.OUT_BF16, False),   # D 7x the operands
+    (4096, 10240, 1024, mx.OUT_F32, True),    # 16-bit D would not fill it
+    (4096, 10240, 1024, mx.OUT_F16, False),
+    (2048, 28672, 1024, mx.OUT_F16, False)])  # D 4x the operands
+def test_rule(M, N, K, out_type, want):
+    Kp = mx.kpad(K)
+    assert mx.splitk_segments(M, N, Kp) == 1
+    assert mx.streams_output(out_type, M, N, Kp, mx.packed_bytes(Kp)) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,out_type", [(8192, 8192, 1024, mx.OUT_BF16),
+                                            (4096, 10240, 960, mx.OUT_F32)])
+def test_equals_direct_kernel(M, N, K, out_type):
+    from gpu_util import DevProblem, run_direct, run_routed
+    p = checks.spread_scales(mx.make_problem(M, N, K, seed=M + N + K), seed=K)
+    assert mx.streams_output(out_type, M, N, p.Kp, p.a_row_bytes)
+    dp = DevProblem(p, mx.choose_tile(M, N, p.Kp))
+    assert (run_routed(dp, out_type).view("u4") == run_direct(dp, out_type).view("u4")).all()
