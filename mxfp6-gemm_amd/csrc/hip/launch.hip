@@ -194,7 +194,11 @@ extern "C" int mxfp6_hip_quantize_rows(const float* x, int rows, int cols, int n
                                        rows32, so));
     }
     const dim3 grid((unsigned)((size_t)rows_out * chunks));
-    return status_of(launch_kernel(v4 ? prep_rows_kernel<true> : prep_rows_kernel<false>, grid,
+    // fewer waves a CU once there are more than 32 for each (1024 x 16128, 32 a CU: 14.6 us against
+    // 14.4; 512 x 16128: 9.2 against 8.7; above, prep_kernel.hpp)
+    const int reported = mxfp6_hip_device_cus();
+    const bool few = (size_t)rows_out * chunks > 32 * (size_t)(reported > 0 ? reported : 256);
+    return status_of(launch_kernel(few ? prep_rows_kernel<true> : prep_rows_kernel<false>, grid,
                                    dim3(64), st, x, cols, nblk, po, so, chunks, rows));
 }
 
@@ -202,7 +206,12 @@ extern "C" int mxfp6_hip_prepare_b(const float* B, int K, int N, int Kp, int gro
                                    uint8_t* tiled, void* stream) {
     const int NG = rows_in_groups(N, group);
     const unsigned nchunks = (unsigned)((NG + PREP_THREADS - 1) / PREP_THREADS), kchunks = (unsigned)(Kp / 32);
-    return status_of(launch_kernel(prep_b_kernel, dim3(nchunks * kchunks), dim3(PREP_THREADS),
+    // B and its codes against half of the 256 MiB last-level cache
+    const double half = 128.0 * (1 << 20), values = (double)K * N;
+    auto k = 4 * values < half     ? prep_b_kernel<false, false>
+             : 0.75 * values < half ? prep_b_kernel<true, false>
+                                    : prep_b_kernel<true, true>;
+    return status_of(launch_kernel(k, dim3(nchunks * kchunks), dim3(PREP_THREADS),
                                    static_cast<hipStream_t>(stream), B, K, N, NG, Kp, group,
                                    static_cast<uint8_t*>(bsh), tiled, (int)nchunks));
 }

@@ -27,9 +27,9 @@
 // scale written):
 //   prep_rows_kernel  row-major float [rows][cols] -> packed rows (+ zero tail up to row_bytes) and
 //                     scales, raw [rows][scale_cols] (tail columns 127) or tiled at Kp. A
-//                     one-wave workgroup takes 64 consecutive 32-blocks of one row: coalesced
-//                     float4 loads into LDS, then lane l quantises block l; the chunk's 1536
-//                     packed bytes go back through LDS and out as 16-byte stores (6 strided
+//                     one-wave workgroup takes 64 consecutive 32-blocks of one row: 16-byte
+//                     loads, a transpose in registers, then lane l quantises block l; the chunk's
+//                     1536 packed bytes go through LDS and out as 16-byte stores (6 strided
 //                     dword stores per lane before: 82 -> 65 us at 8192 x 8192).
 //   prep_rows_preshuffled_kernel  row-major float A -> the preshuffled operand layout + tiled
 //                     scales: a workgroup stages 32 rows x 4 slabs in LDS, each wave then writes
@@ -158,6 +158,19 @@ __device__ __forceinline__ void put_block(const PackedOut& po, const ScaleOut& s
     }
 }
 
+// Exchanges the upper half wave of a with the lower half of b; and, in each half, the upper 16 lanes of a
+// with the lower 16 of b.
+__device__ __forceinline__ void swap_halves(float& a, float& b) {
+    const v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap_rows(float& a, float& b) {
+    const v2u r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+
 // One wave per workgroup (no barrier across waves); workgroup = task (row r, chunk), row-major,
 // r < rows_out, chunk < chunks = ceil(vblk / 64) with vblk = ceil(cols / 32) the blocks holding
 // values. A task quantises the value blocks 64 chunk .. +63 of its row (lane l: block
@@ -166,14 +179,23 @@ __device__ __forceinline__ void put_block(const PackedOut& po, const ScaleOut& s
 // rows that complete the last 32-row block of a preshuffled output and the last scale group of a
 // tiled one (zero codes, scale 127). Block c of row r (c < nblk) writes the codes of values
 // 32c .. 32c+31 (zero past cols) as put_block places them, and the scale column c if
-// c < so.ncols. V4: cols % 4 == 0 and x 16-byte aligned (float4 loads);
-// otherwise one float per lane per load.
-template <bool V4>
+// c < so.ncols.
+// The values come straight into registers: lane 16 j + i loads the 32-byte piece j of the blocks
+// 16 g + i, g = 0 .. 3 (16-byte loads, four lanes on a block's 128 bytes), and a 4 x 4 transpose of
+// (piece, block group) between lanes and registers, two exchanges of wave halves and quarters per
+// value, leaves lane l the whole of block l. A wave's LDS is then only its 1.5 KiB of codes, and
+// FEW can bound the waves in flight instead: at the rates of a large input the time is the
+// memory's (321 MB at 8192 x 8192), which runs faster with 12 waves a CU (each with 8 KiB of loads)
+// than with as many as fit: 67.3 us (16 waves, the values transposed through 8.4 KiB of LDS),
+// 66.6 with 32, 60.8 with 12, 72.3 with 6; 2048 x 16128 36.2 -> 33.9. Nontemporal loads lose
+// here (67): the input has often just been written.
+template <bool FEW>
 __global__ void __launch_bounds__(64)
     prep_rows_kernel(const float* __restrict__ x, int cols, int nblk, PackedOut po, ScaleOut so,
                      int chunks, int rows) {
     constexpr int BPW = PREP_BLKS_PER_WAVE;  // blocks per task, one per lane
-    __shared__ __attribute__((aligned(16))) float stage[BPW * 33];
+    // the codes of the task; FEW: padded to a twelfth of a CU's 160 KiB
+    __shared__ __attribute__((aligned(16))) uint32_t ob[FEW ? 13312 / 4 : BPW * 6];
     const int lane = threadIdx.x;
     const int r = (int)(blockIdx.x / (unsigned)chunks);
     const int chunk = (int)(blockIdx.x - (unsigned)r * chunks);
@@ -181,42 +203,45 @@ __global__ void __launch_bounds__(64)
     const int blk0 = chunk * BPW;
     const int vblk = (cols + 31) / 32;
     const float* xr = x + (size_t)r * cols;
-    // coalesced loads of the task's values, block-padded in LDS
-    if (data) {
-        if constexpr (V4) {
+    const int i = lane & 15, j = lane >> 4;
+    float v[4][8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int p = 4 * (lane + 64 * j);  // value index within the task's range
-                const int b = p >> 5, i = p & 31, e = blk0 * 32 + p;
-                v4f v = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (e < cols) v = *reinterpret_cast<const v4f*>(xr + e);
-                stage[b * 33 + i] = v[0];
-                stage[b * 33 + i + 1] = v[1];
-                stage[b * 33 + i + 2] = v[2];
-                stage[b * 33 + i + 3] = v[3];
+    for (int g = 0; g < 4; g++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int e = (blk0 + 16 * g + i) * 32 + 8 * j + 4 * h;
+            v4f_a4 q = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (data && e + 3 < cols) {
+                q = *reinterpret_cast<const v4f_a4*>(xr + e);
+            } else if (data) {
+#pragma unroll
+                for (int k = 0; k < 3; k++)
+                    if (e + k < cols) q[k] = xr[e + k];
             }
-        } else {
-#pragma unroll 8
-            for (int j = 0; j < 32; j++) {
-                const int p = lane + 64 * j, e = blk0 * 32 + p;
-                stage[(p >> 5) * 33 + (p & 31)] = e < cols ? xr[e] : 0.0f;
-            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[g][4 * h + k] = q[k];
         }
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        swap_halves(v[0][k], v[2][k]);
+        swap_halves(v[1][k], v[3][k]);
+        swap_rows(v[0][k], v[1][k]);
+        swap_rows(v[2][k], v[3][k]);
     }
-    __syncthreads();
     const int c = blk0 + lane;
-    // a whole chunk of value blocks into 16-byte aligned row-major rows: staged in LDS and stored
-    // as 16-byte contiguous pieces
+    uint32_t w[6] = {0, 0, 0, 0, 0, 0};
+    int code = 127;
+    if (data && c < vblk) {
+        float u[32];
+#pragma unroll
+        for (int k = 0; k < 32; k++) u[k] = v[k >> 3][k & 7];
+        code = quant32(u, w);
+    }
+    // a whole chunk of value blocks into row-major rows of a multiple of 16 bytes: through LDS and
+    // stored as 16-byte contiguous pieces
     const bool full = po.k64n == 0 && data && (po.row_bytes % 16) == 0 && blk0 + BPW <= vblk &&
                       (size_t)24 * (blk0 + BPW) <= po.row_bytes;
     if (full) {
-        uint32_t w[6];
-        float v[32];
-#pragma unroll
-        for (int i = 0; i < 32; i++) v[i] = stage[lane * 33 + i];
-        const int code = quant32(v, w);
-        __syncthreads();
-        uint32_t* ob = reinterpret_cast<uint32_t*>(stage);
 #pragma unroll
         for (int d = 0; d < 6; d++) ob[lane * 6 + d] = w[d];
         __syncthreads();
@@ -234,14 +259,6 @@ __global__ void __launch_bounds__(64)
                 so.p[(size_t)r * so.ncols + c] = (uint8_t)code;
         }
     } else if (c < nblk) {
-        uint32_t w[6] = {0, 0, 0, 0, 0, 0};
-        int code = 127;
-        if (data && c < vblk) {
-            float v[32];
-#pragma unroll
-            for (int i = 0; i < 32; i++) v[i] = stage[lane * 33 + i];
-            code = quant32(v, w);
-        }
         put_block(po, so, r, c, data, w, code);
     }
     if (chunk == chunks - 1) {
@@ -324,9 +341,20 @@ __global__ void __launch_bounds__(64 * PSH_SLABS)
 // Columns N .. NG-1 (NG = N rounded up to whole scale groups of 32 * group columns) are zero
 // columns: they complete the last 32-column tile of bsh and the last scale group. Values past K
 // in the last 32-block are zero.
+// FEW (large B): four workgroups a CU instead of eight, bounded by an unused quarter of its LDS, and
+// nontemporal loads: with fewer rows' pieces in flight the memory serves them faster, and B is not
+// read again (8192 x 4096 34.0 -> 28.0 us, 8192 x 8192 62.0 -> 52.3, 8192 x 14336 107.5 -> 95.9;
+// FEW alone 31.4, 58.1 and 103.9; B that the last-level cache may hold loses by nontemporal loads,
+// 8192 x 2048 12.8 -> 15.2). NTS stores the codes nontemporally too, where they would fill half that
+// cache: 8192 x 28672 218.9 -> 205.0 with FEW, 198.5 with both.
+template <bool FEW, bool NTS>
 __global__ void __launch_bounds__(PREP_THREADS)
     prep_b_kernel(const float* __restrict__ B, int K, int N, int NG, int Kp, int group,
                   uint8_t* __restrict__ bsh, uint8_t* __restrict__ tiled, int nchunks) {
+    if constexpr (FEW) {
+        __shared__ uint32_t lds_quarter[40960 / 4];
+        asm volatile("" ::"s"((uint32_t)(uintptr_t)lds_quarter));
+    }
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int kc = (int)(blockIdx.x / nchunks), nb = (int)(blockIdx.x - (unsigned)kc * nchunks);
     const int n = nb * PREP_THREADS + wave * 64 + lane;
@@ -339,14 +367,22 @@ __global__ void __launch_bounds__(PREP_THREADS)
         const float* src = B + (size_t)32 * c * N + n;
         const int kv = min(32, K - 32 * c);  // values of this block
 #pragma unroll
-        for (int i = 0; i < 32; i++) v[i] = i < kv ? src[(size_t)i * N] : 0.0f;
+        for (int i = 0; i < 32; i++)
+            v[i] = i >= kv ? 0.0f : FEW ? __builtin_nontemporal_load(src + (size_t)i * N) : src[(size_t)i * N];
         code = quant32(v, w);
     }
     if (n < (N + 31) / 32 * 32) {
         const int k64n = Kp / 64, t = (n & 31) + ((c & 1) << 5);
         uint8_t* tile = bsh + ((size_t)(n >> 5) * k64n + (c >> 1)) * OPBLK_BYTES;
-        *reinterpret_cast<v4i*>(tile + 16 * t) = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-        *reinterpret_cast<v2i*>(tile + 1024 + 8 * t) = v2i{(int)w[4], (int)w[5]};
+        const v4i lo = {(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+        const v2i hi = {(int)w[4], (int)w[5]};
+        if constexpr (NTS) {
+            __builtin_nontemporal_store(lo, reinterpret_cast<v4i*>(tile + 16 * t));
+            __builtin_nontemporal_store(hi, reinterpret_cast<v2i*>(tile + 1024 + 8 * t));
+        } else {
+            *reinterpret_cast<v4i*>(tile + 16 * t) = lo;
+            *reinterpret_cast<v2i*>(tile + 1024 + 8 * t) = hi;
+        }
     }
     put_tiled_scale(tiled, n, c, group, Kp / 192, code);
 }
