@@ -419,6 +419,8 @@ int wide_launch_t(const mxfp6_launch_desc* d, hipStream_t st) {
     const bool mask = d->M % G::MT != 0 || d->N % G::NT != 0;
     // the swizzled staging of row-major A: unmasked tiles, plain stores
     if (d->a_layout == MXFP6_A_ROWS_SWIZZLED && (mask || d->out_stream)) return 2;
+    // a grid that leaves many CUs idle runs as 128-row bands of the stream kernel
+    if (const int wn = band_waves(d)) return band_launch<KT, SPLIT>(d, wn, st);
     const uint8_t* A = static_cast<const uint8_t*>(d->A);
     if (d->a_layout == MXFP6_A_REPACK) {
         if (repack_rows_launch(A, d->A_row_bytes, d->M, d->Kp / 64, static_cast<uint8_t*>(d->Ash),

@@ -1,5 +1,5 @@
-// Stream kernels of libmxfp6gemm for gfx950: the skinny tiles (32 and 64 rows) on row-major A, B read
-// once and straight into registers.
+// Stream kernels of libmxfp6gemm for gfx950: the skinny tiles (32 and 64 rows) and, on small grids, the
+// wide tiles (as 128-row bands) on row-major A, B read straight into registers.
 //
 // A workgroup computes an MT x NT tile of D with MT = 32 MB and NT = 32 NPW WN: WN computing waves
 // side by side, each owning all MT rows and 32 NPW columns, and one copying wave. (MB, NPW) is the
@@ -28,6 +28,14 @@
 // NT: B's loads are nontemporal where B exceeds half the last-level cache and is read by one tile
 // row: 44.8 -> 39.1 us at 64 x 28672 x 8192 (B 176 MB), while B that would have stayed in the cache
 // loses (64 x 8192 x 8192, B 50 MB: 20.9 -> 31.4 us).
+// BAND (WN = 0 in the template; 128 rows, scale groups of four row blocks): a wave owns 128 rows and
+// one 32-column block, byte blk % npw of its scale group of npw blocks, so that the launch can
+// choose how many columns a workgroup takes (2 to 5 computing waves, all in one round of the CUs)
+// whatever the tile: same bits as the wide kernel's tiles of that grouping. Two copying waves share
+// a chunk's copies, and the A operands are read a slab ahead (a K-tile's would not fit the
+// registers). Against the wide kernel on a grid that leaves CUs idle each CU in use has fewer cache
+// lines to fetch: per K-tile 26 KB of A and 5.4 KB a wave, where a 128 x 256 tile takes 76 KB
+// (256 x 18432 x 12288, 144 workgroups of 128 x 256 or 232 of five waves: 88.1 -> 66.6 us).
 // MASK (ragged M or N): rows past M repeat the last one, blocks and scale groups past the end the last
 // that exists; stores are masked.
 #pragma once
@@ -43,19 +51,24 @@ namespace mxfp6_dev {
 template <int MB_, int NPW_, int WN_>
 struct StreamGeom {
     static constexpr int MB = MB_, NPW = NPW_, WN = WN_;
+    static constexpr bool BAND = WN == 0;                       // WN given by the launch
+    static constexpr int NCW = BAND ? 2 : 1;                    // copying waves
+    static constexpr int MAXWN = BAND ? 5 : WN;
     static constexpr int L = 2;                                 // K-tiles of B in flight
     static constexpr int CK = 2;                                // K-tiles of A a chunk
     static constexpr int NB = 3;                                // chunk buffers
     static constexpr int MT = 32 * MB, NT = 32 * NPW * WN;
-    static constexpr int THREADS = 64 * (WN + 1);
+    static constexpr int THREADS = 64 * (MAXWN + NCW);
     static constexpr int ROW = 9 * CK + 1;                      // 16-byte LDS pieces a row, one of padding
     static constexpr int PIECES = MT * ROW;
     static constexpr int COPIES = (PIECES + 63) / 64;           // wave copies of a chunk's rows
-    static constexpr int OPS = COPIES + CK;                     // and one of each K-tile's scales
-    static constexpr int CST = OPS * 1024;                      // LDS buffer stride
+    // operations of a copying wave for a chunk: its rows' copies and one of a K-tile's scales
+    static constexpr int OPS = (COPIES + CK) / NCW;
+    static constexpr int CST = (COPIES + CK) * 1024;            // LDS buffer stride
     static constexpr int LDS = NB * CST;
     static constexpr int PASS = 2;                              // K-tiles of a pass of the K loop
     static_assert(PASS % CK == 0 && PASS % L == 0 && PASS % 2 == 0, "ring positions are constants");
+    static_assert(COPIES % NCW == 0 && CK % NCW == 0, "copies shared evenly");
     static_assert((NB - 1) * OPS <= 63, "vmcnt range");
     static_assert(LDS <= 160 * 1024, "LDS budget");
 };
@@ -72,13 +85,13 @@ __device__ __forceinline__ void stream_tail(int left, F&& f) {
 }
 
 template <int MB_, int NPW_, int WN_, int XG, typename OutT, bool SPLIT, bool MASK, bool NTB>
-__global__ void __launch_bounds__(64 * (WN_ + 1), 1)
+__global__ void __launch_bounds__(64 * (WN_ == 0 ? 7 : WN_ + 1), 1)
     stream_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ Bsh,
                   const uint8_t* __restrict__ sA, const uint8_t* __restrict__ sB,
                   OutT* __restrict__ D, float* __restrict__ ws, int M, int N, int Kp,
-                  int A_row_bytes, int S) {
+                  int A_row_bytes, int S, int npw) {
     using G = StreamGeom<MB_, NPW_, WN_>;
-    constexpr int MT = G::MT, NT = G::NT, MB = G::MB, NPW = G::NPW, WN = G::WN, L = G::L;
+    constexpr int MT = G::MT, MB = G::MB, NPW = G::NPW, NCW = G::NCW, L = G::L;
     constexpr int CK = G::CK, NB = G::NB;
     constexpr int AUX = NTB ? 2 : 0;  // cache policy of the B loads (2: nontemporal)
     __shared__ __attribute__((aligned(1024))) char lds[G::LDS];
@@ -96,16 +109,19 @@ __global__ void __launch_bounds__(64 * (WN_ + 1), 1)
     if (SPLIT) split_segment(k_tiles, S, wg_z, kt0, nkt);
     const int kt_last = kt0 + nkt - 1;
 
-    if (wave == WN) {
+    const int WN = G::BAND ? (int)(blockDim.x >> 6) - NCW : G::WN;
+
+    if (wave >= WN) {
         // the copying wave: copy i moves LDS piece p = 64 i + l of a chunk (16 bytes, lane l) from
         // piece p % ROW of row p / ROW; the padding piece is not copied, nor are the pieces past the
         // segment's end. Every copy has at least one lane to copy, so a chunk is OPS operations.
         const int rows = MASK ? min(MT, M - wg_m * MT) : MT;
         const uint8_t* a_tile = A + (size_t)wg_m * MT * A_row_bytes + (size_t)kt0 * (SUBS * SLAB_BYTES);
-        uint32_t voff[G::COPIES];
+        const int cw = wave - WN;  // copies cw, cw + NCW, ...
+        uint32_t voff[G::COPIES / NCW];
 #pragma unroll
-        for (int i = 0; i < G::COPIES; i++) {
-            const int p = i * 64 + lane, row = p / G::ROW, col = p - row * G::ROW;
+        for (int i = 0; i < G::COPIES / NCW; i++) {
+            const int p = (i * NCW + cw) * 64 + lane, row = p / G::ROW, col = p - row * G::ROW;
             voff[i] = p < G::PIECES && col < 9 * CK
                           ? (uint32_t)((MASK ? min(row, rows - 1) : row) * A_row_bytes + 16 * col)
                           : ~0u;
@@ -117,21 +133,22 @@ __global__ void __launch_bounds__(64 * (WN_ + 1), 1)
         const int nch = (nkt + CK - 1) / CK;
         auto copy = [&](int ch) {
             const uint8_t* src = a_tile + (size_t)ch * (CK * SUBS * SLAB_BYTES);
-            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + ch % NB * G::CST);
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + ch % NB * G::CST + cw * 1024);
             const int kts = min(CK, nkt - ch * CK);
             if (kts == CK) {
 #pragma unroll
-                for (int i = 0; i < G::COPIES; i++)
-                    if (voff[i] != ~0u) dma16(dst + i * 1024, src, voff[i]);
+                for (int i = 0; i < G::COPIES / NCW; i++)
+                    if (voff[i] != ~0u) dma16(dst + i * NCW * 1024, src, voff[i]);
             } else {
 #pragma unroll
-                for (int i = 0; i < G::COPIES; i++) {
-                    const int col = (i * 64 + lane) % G::ROW;
-                    if (voff[i] != ~0u && col < 9 * kts) dma16(dst + i * 1024, src, voff[i]);
+                for (int i = 0; i < G::COPIES / NCW; i++) {
+                    const int col = ((i * NCW + cw) * 64 + lane) % G::ROW;
+                    if (voff[i] != ~0u && col < 9 * kts) dma16(dst + i * NCW * 1024, src, voff[i]);
                 }
             }
-            const uint32_t sdst = __builtin_amdgcn_readfirstlane(dst + G::COPIES * 1024);
-            for (int t = 0; t < CK; t++)
+            const uint32_t sdst =
+                __builtin_amdgcn_readfirstlane(lds0 + ch % NB * G::CST + G::COPIES * 1024);
+            for (int t = cw; t < CK; t += NCW)
                 dma12_at<0>(sdst + t * 1024, sa_grp + (size_t)(ch * CK + min(t, kts - 1)) * 768, sc_voff);
         };
         for (int ch = 0; ch < NB && ch < nch; ch++) copy(ch);
@@ -156,12 +173,19 @@ __global__ void __launch_bounds__(64 * (WN_ + 1), 1)
     rsrc_t b_rs[NPW];
 #pragma unroll
     for (int ni = 0; ni < NPW; ni++) {
-        int blk = wg_n * (NT / 32) + wave * NPW + ni;
+        int blk = (wg_n * WN + wave) * NPW + ni;
         if (MASK) blk = min(blk, b_blk_last);
         b_rs[ni] = raw_rsrc(opaque_gptr(Bsh + (size_t)blk * k64n * OPBLK_BYTES));
     }
-    int gb = wg_n * WN + wave;
-    if (MASK) gb = min(gb, ((N + 31) / 32 + NPW - 1) / NPW - 1);
+    // the wave's B scale group; BAND: its one block is byte b_shift / 8 of a group of npw blocks
+    int gb = wg_n * WN + wave, b_shift = 0;
+    if constexpr (G::BAND) {
+        const int blk = min(gb, b_blk_last);
+        gb = blk / npw;
+        b_shift = 8 * (blk - gb * npw);
+    } else if (MASK) {
+        gb = min(gb, ((N + 31) / 32 + NPW - 1) / NPW - 1);
+    }
     const rsrc_t sb_rs = raw_rsrc(opaque_gptr(sB + (size_t)gb * k_tiles * 64 * 12));
     const int v_b0 = (int)opaque_v(16 * lane), v_b1 = (int)opaque_v(1024 + 8 * lane);
     const int v_sc = (int)opaque_v(12 * lane);
@@ -204,47 +228,76 @@ __global__ void __launch_bounds__(64 * (WN_ + 1), 1)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     }
-    // A operands and scales of a K-tile, two sets
-    v8i RA[2][SUBS][MB];
+    // A operands, two sets: of a K-tile, or (BAND, whose sets are larger) of a slab; A scales of a
+    // K-tile, two sets
+    constexpr int US = G::BAND ? 1 : SUBS;
+    v8i RA[2][US][MB];
     v3i sc_a[2];
-    auto read_a = [&](auto qq, auto tt, int buf) {
+    // the A scales of K-tile KT of the chunk in buffer buf to set Q
+    auto read_sc = [&](auto qq, auto tt, int buf) {
         constexpr int Q = decltype(qq)::value, KT = decltype(tt)::value;
-        const uint32_t base = opaque_v(a_rd + buf * G::CST);
         sc_a[Q] = *reinterpret_cast<const __attribute__((address_space(3))) v3i*>(
             lds3 + opaque_v(16 * lane + buf * G::CST) + (G::COPIES + KT) * 1024);
+    };
+    // and the A operands of its slabs s0 .. s0 + US - 1
+    auto read_a = [&](auto qq, auto tt, int s0, int buf) {
+        constexpr int Q = decltype(qq)::value, KT = decltype(tt)::value;
+        const uint32_t base = opaque_v(a_rd + buf * G::CST);
 #pragma unroll
-        for (int s = 0; s < SUBS; s++)
+        for (int s = 0; s < US; s++)
 #pragma unroll
             for (int mi = 0; mi < MB; mi++) {
                 const v6i_a8 x = *reinterpret_cast<const __attribute__((address_space(3))) v6i_a8*>(
-                    lds3 + base + mi * 32 * G::ROW * 16 + KT * SUBS * SLAB_BYTES + s * SLAB_BYTES);
+                    lds3 + base + mi * 32 * G::ROW * 16 + KT * SUBS * SLAB_BYTES + (s0 + s) * SLAB_BYTES);
                 RA[Q][s][mi] = __builtin_shufflevector(x, x, 0, 1, 2, 3, 4, 5, -1, -1);
             }
     };
+    using I0 = std::integral_constant<int, 0>;
     ring_barrier();
-    read_a(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, 0);
+    read_sc(I0{}, I0{}, 0);
+    read_a(I0{}, I0{}, 0, 0);
     int buf = 0;
     auto ktile = [&](int c, auto tt) {
-        constexpr int T = decltype(tt)::value % L, Q = decltype(tt)::value % 2;
-        constexpr int NEXT = (decltype(tt)::value + 1) % CK;
-        if constexpr (NEXT == 0) {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            ring_barrier();
-            buf = buf == NB - 1 ? 0 : buf + 1;
+        constexpr int T = decltype(tt)::value % L, P = decltype(tt)::value % 2;
+        constexpr int KT = decltype(tt)::value % CK, NEXT = (KT + 1) % CK;
+        using NextC = std::integral_constant<int, NEXT>;
+        using ScC = std::integral_constant<int, 1 - P>;
+        // K-tile c + 1 is read from here on: at a chunk's end once it has landed
+        auto next_ktile = [&] {
+            if constexpr (NEXT == 0) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                ring_barrier();
+                buf = buf == NB - 1 ? 0 : buf + 1;
+            }
+            read_sc(ScC{}, NextC{}, buf);
+        };
+        if constexpr (US == SUBS) {
+            next_ktile();
+            read_a(ScC{}, NextC{}, 0, buf);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        read_a(std::integral_constant<int, 1 - Q>{}, std::integral_constant<int, NEXT>{}, buf);
-        __builtin_amdgcn_sched_barrier(0);
         const int kt_next = min(kt0 + c + L, kt_last);
-        const v3i ca = sc_a[Q], cb = sc_b[T];
-#pragma unroll
-        for (int s = 0; s < SUBS; s++) {
+        const v3i ca = sc_a[P], cb = sc_b[T];
+        static_for<SUBS>([&](auto ss) {
+            constexpr int s = decltype(ss)::value;
+            constexpr int Q = US == SUBS ? P : (P + s) % 2;  // 3 c + s, modulo 2
+            if constexpr (US == 1) {
+                if constexpr (s + 1 < SUBS) {
+                    read_a(std::integral_constant<int, 1 - Q>{}, std::integral_constant<int, KT>{}, s + 1, buf);
+                } else {
+                    next_ktile();
+                    read_a(std::integral_constant<int, 1 - Q>{}, NextC{}, 0, buf);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
             const int sa = s == 0 ? ca.x : s == 1 ? ca.y : ca.z;
-            const int sb = s == 0 ? cb.x : s == 1 ? cb.y : cb.z;
+            int sb = s == 0 ? cb.x : s == 1 ? cb.y : cb.z;
+            if constexpr (G::BAND) sb = (int)((uint32_t)sb >> b_shift);
 #pragma unroll
             for (int ni = 0; ni < NPW; ni++) {
 #pragma unroll
                 for (int mi = 0; mi < MB; mi++)
-                    wide_mfma<MB, NPW>(acc, mi, ni, RA[Q][s][mi], RB[T][s][ni], sa, sb);
+                    wide_mfma<MB, NPW>(acc, mi, ni, RA[Q][US == SUBS ? s : 0][mi], RB[T][s][ni], sa, sb);
                 __builtin_amdgcn_sched_barrier(0);
                 load_b(RB[T][s][ni], ni, kt_next, s);
                 asm volatile("" ::: "memory");
@@ -255,7 +308,7 @@ __global__ void __launch_bounds__(64 * (WN_ + 1), 1)
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
-        }
+        });
     };
     // Whole passes, then the K-tiles left. No exit inside a pass: where it met the loop's back edge
     // the compiler would wait for loads just issued. For the same reason a K-tile's scale load comes
@@ -266,7 +319,7 @@ __global__ void __launch_bounds__(64 * (WN_ + 1), 1)
     stream_tail<0, PASS>(nkt - c, [&](auto tt) { ktile(c + decltype(tt)::value, tt); });
     const int le = lane_id();
     store_tile<MB, NPW, OutT, SPLIT, MASK>(acc, D, ws, M, N, wg_m * MT + 4 * (le >> 5),
-                                           wg_n * NT + wave * NPW * 32 + (le & 31), le, wg_z);
+                                           (wg_n * WN + wave) * NPW * 32 + (le & 31), le, wg_z);
 }
 
 // One launch for a tile of grouping (MB, NPW), four computing waves wide as the router counts it.
@@ -295,7 +348,7 @@ hipError_t stream_launch_w(const mxfp6_launch_desc* d, bool ntb, hipStream_t st)
     return launch_kernel(k, grid, dim3(G::THREADS), st, static_cast<const uint8_t*>(d->A),
                          static_cast<const uint8_t*>(d->Bsh), d->sA, d->sB,
                          SPLIT ? nullptr : static_cast<KT*>(d->D), SPLIT ? d->ws : nullptr, d->M,
-                         d->N, d->Kp, d->A_row_bytes, SPLIT ? d->splits : 1);
+                         d->N, d->Kp, d->A_row_bytes, SPLIT ? d->splits : 1, NPW);
 }
 
 // Returns 0, or 2 when the launch fails.
@@ -323,6 +376,44 @@ int stream_launch(const mxfp6_launch_desc* d, hipStream_t st) {
         else
             e = stream_launch_w<MB, NPW, 4, KT, SPLIT>(d, ntb, st);
     }
+    return e == hipSuccess ? 0 : 2;
+}
+
+// Computing waves of the BAND launch that runs a wide tile's plan on row-major A, or 0 where the wide
+// kernel is the better one: the fewest with which the plan's workgroups run in one round of the
+// CUs. Up to four were never slower than the wide kernel on 43 measured shapes, three operand sets in
+// turn (three waves 2048 x 1152 x 2128 1.25x, 128 x 24576 x 4096 1.52x; four 512 x 8192 x 2048 1.00x,
+// 1203 x 2560 x 1408 1.12x, 128 x 2048 x 50116 in 16 segments 1.16x); five only where B is no small
+// part of the 256 MiB last-level cache (57 MB 1.03-1.08x unsplit, 0.90 split; 75 MB 1.29x, 126 MB
+// in two segments 1.18x, 170 MB 1.32x; 28 MB 0.91, 42 MB 1.00), for there the wide kernel's loads, one
+// K-tile ahead, wait on HBM; six lost but for one shape (682 x 1280 x 27520 in 6 segments 0.76, 256 x
+// 7040 x 9920 in 3 0.89; 128 x 6016 x 18944 in 8 1.15x). Segments of fewer than eight K-tiles keep the
+// wide kernel, which has short paths for them.
+inline int band_waves(const mxfp6_launch_desc* d) {
+    if (d->a_layout != MXFP6_A_ROWS || d->mpw != 4 || d->out_stream || d->Kp / 192 < 8 * d->splits)
+        return 0;
+    const int reported = mxfp6_hip_device_cus();
+    const long cus = reported > 0 ? reported : 256;
+    const long rows = (long)((d->M + 127) / 128) * d->splits, blks = (d->N + 31) / 32;
+    const bool large_b = (double)d->N * (d->Kp / 4 * 3) > 64.0 * (1 << 20);
+    for (int wn = 2; wn <= (large_b ? 5 : 4); wn++)
+        if (rows * ((blks + wn - 1) / wn) <= cus) return wn;
+    return 0;
+}
+
+// Returns 0, or 2 when the launch fails.
+template <typename KT, bool SPLIT>
+int band_launch(const mxfp6_launch_desc* d, int wn, hipStream_t st) {
+    using G = StreamGeom<4, 1, 0>;
+    const bool ntb = d->M <= 128 && (double)d->N * (d->Kp / 4 * 3) > 128.0 * (1 << 20);
+    const dim3 grid((unsigned)((d->M + 127) / 128), (unsigned)((d->N + 32 * wn - 1) / (32 * wn)),
+                    (unsigned)d->splits);
+    const hipError_t e = launch_kernel(
+        ntb ? stream_kernel<4, 1, 0, 4, KT, SPLIT, true, true>
+            : stream_kernel<4, 1, 0, 4, KT, SPLIT, true, false>,
+        grid, dim3(64 * (wn + G::NCW)), st, static_cast<const uint8_t*>(d->A),
+        static_cast<const uint8_t*>(d->Bsh), d->sA, d->sB, SPLIT ? nullptr : static_cast<KT*>(d->D),
+        SPLIT ? d->ws : nullptr, d->M, d->N, d->Kp, d->A_row_bytes, SPLIT ? d->splits : 1, d->npw);
     return e == hipSuccess ? 0 : 2;
 }
 
