@@ -131,8 +131,10 @@ int mxfp6_gemm_explicit(int out_type, int M, int N, int Kp, const int tile[4], i
                         const uint8_t* dsB, void* dD, int A_row_bytes, void* ws, size_t ws_bytes,
                         void* stream);
 
-/* Whether gemm() repacks A for (M, N, Kp) when its workspace allows. No counterpart in the
- * reference (its kernels read A row-major). */
+/* Whether the routed plan for (M, N, Kp) has room for a repacked A in its preferred workspace (gemm()
+ * repacks A there, or, on 32- and 64-row tiles with many workgroups, reads the rows as they are
+ * where that is faster: the same bits). No counterpart in the reference (its kernels read A
+ * row-major). */
 int mxfp6_gemm_repacks_a(int M, int N, int Kp);
 
 /* Measured plan selection. No counterpart in the reference (its router is a fixed rule).

@@ -164,6 +164,10 @@ extern "C" int mxfp6_hip_has_tile(int MT, int NT, int mpw, int npw) {
     return tile_supported(MT, NT, mpw, npw) ? 1 : 0;
 }
 
+extern "C" int mxfp6_hip_prefers_rows(int M, int N, int splits, int MT) {
+    return MT <= 64 && skinny_runs_wide(M, N, splits, true) ? 1 : 0;
+}
+
 // Rows of the tiled scale layout: dim rounded up to whole groups of 32 * group rows.
 static int rows_in_groups(int dim, int group) {
     return (dim + 32 * group - 1) / (32 * group) * (32 * group);

@@ -387,14 +387,6 @@ int slab_launch_t(const mxfp6_launch_desc* d, hipStream_t st) {
     return e == hipSuccess ? 0 : 2;
 }
 
-// The skinny tiles: row-major A on the stream kernel, A repacked or preshuffled on the slab kernel
-// with one wave row and four wave columns.
-template <int MT, int NT, typename KT, bool SPLIT>
-int skinny_launch(const mxfp6_launch_desc* d, hipStream_t st) {
-    if (d->a_layout == MXFP6_A_ROWS) return stream_launch<MT / 32, NT / 128, KT, SPLIT>(d, st);
-    return slab_launch_t<MT, NT, 1, 4, 4, 8, KT, SPLIT, false>(d, st);
-}
-
 // The wide tiles (four waves side by side, B straight to registers): the A repack first when
 // asked, MASK when the tile does not divide M x N. Three LDS chunk buffers; XCD groups of 8 tile
 // rows for the 128-row tiles (4 buffers and groups of 4 or 16 rows measured within run-to-run
@@ -436,6 +428,28 @@ int wide_launch_t(const mxfp6_launch_desc* d, hipStream_t st) {
         e = mask ? wide_launch_st<MB, NPW, XG, KT, SPLIT, true, true>(d, A, st)
                  : wide_launch_st<MB, NPW, XG, KT, SPLIT, true, false>(d, A, st);
     return e == hipSuccess ? 0 : 2;
+}
+
+// The skinny tiles: row-major A on the stream kernel, or on 128 x 256 wide tiles that read the skinny
+// tile's scale groups; A repacked or preshuffled on the slab kernel with one wave row and four wave
+// columns. All give the same bits.
+template <int MT, int NT, typename KT, bool SPLIT>
+int skinny_launch(const mxfp6_launch_desc* d, hipStream_t st) {
+    if (d->a_layout != MXFP6_A_ROWS) return slab_launch_t<MT, NT, 1, 4, 4, 8, KT, SPLIT, false>(d, st);
+    if (skinny_runs_wide(d->M, d->N, d->splits, false)) {
+        using G = WideGeom<4, 2, WIDE_NB, false, MT / 32, NT / 128>;
+        const dim3 grid((unsigned)((d->M + G::MT - 1) / G::MT), (unsigned)((d->N + G::NT - 1) / G::NT),
+                        (unsigned)d->splits);
+        return launch_kernel(wide_kernel<4, 2, WIDE_NB, 8, KT, SPLIT, false, true, false, 0, false,
+                                         G::GA, G::GB>,
+                             grid, dim3(G::THREADS), st, static_cast<const uint8_t*>(d->A),
+                             static_cast<const uint8_t*>(d->Bsh), d->sA, d->sB,
+                             SPLIT ? nullptr : static_cast<KT*>(d->D), SPLIT ? d->ws : nullptr, d->M,
+                             d->N, d->Kp, d->A_row_bytes, SPLIT ? d->splits : 1) == hipSuccess
+                   ? 0
+                   : 2;
+    }
+    return stream_launch<MT / 32, NT / 128, KT, SPLIT>(d, st);
 }
 
 // Tile dispatch (declared in slab_run.hpp; instantiated once per (KT, SPLIT) in its own

@@ -68,13 +68,13 @@ namespace mxfp6_dev {
 // MFMA k; (s = 0, k = 0) the scale loads of the next K-tile; the slab's next A copy when k is a
 // copy position; the two loads of B block k / MB when MFMA k was its last use in the slab
 // (k % MB == MB - 1); the LDS read of an A block of the next slab when k is a read position.
-template <int MB_, int NPW_, int NB_, bool SWZ_ = false>
+template <int MB_, int NPW_, int NB_, bool SWZ_ = false, int GA_ = 4, int GB_ = NPW_>
 struct WideGeom {
     static constexpr int MB = MB_, NPW = NPW_, NB = NB_;
     static constexpr bool SWZ = SWZ_;                            // 12-byte units, swizzled rows
     static constexpr int MT = 32 * MB, NT = 4 * 32 * NPW, NWAVES = 4, THREADS = 256;
-    static constexpr int GA = MB < 4 ? MB : 4;                   // A scale group (blocks)
-    static constexpr int NGA = MB / GA;                          // A scale groups per tile
+    static constexpr int GA = GA_, NGA = MB / GA;                // A scale group (blocks), per tile
+    static constexpr int GB = GB_, NGB = NPW / GB;               // B scale group, per wave
     static constexpr int NMF = MB * NPW;                         // MFMAs per wave per slab
     static constexpr int NSET = MB <= 4 ? 3 : 2;                 // A operand register sets
     static constexpr int CHUNK = MT * SUBS * SLAB_BYTES;         // one K-tile of A
@@ -92,7 +92,7 @@ struct WideGeom {
     static constexpr bool b_load_at(int k) { return k % MB == MB - 1; }
     // MFMA after which the read of A block i of the next slab is issued
     static constexpr int read_k(int i) { return NSET == 3 ? NMF / 2 + i : i * (NMF / MB); }
-    static constexpr int ops_in_slab(int s) { return (s == 0 ? NGA + 1 : 0) + cps(s) + 2 * NPW; }
+    static constexpr int ops_in_slab(int s) { return (s == 0 ? NGA + NGB : 0) + cps(s) + 2 * NPW; }
     static constexpr int ops_in_ktile() { return ops_in_slab(0) + ops_in_slab(1) + ops_in_slab(2); }
     static constexpr int b_ops_from(int k0) {
         int n = 0;
@@ -107,18 +107,20 @@ struct WideGeom {
                                       ops_in_slab(0) + ops_in_slab(1);
     // In the prologue: after chunk 0's copies, those of chunks 1 .. NB - 2, the scale loads of
     // K-tile 0 and the B loads of its three slabs.
-    static constexpr int PRO_WAIT = (NB - 2) * A_ISS + NGA + 1 + SUBS * 2 * NPW;
+    static constexpr int PRO_WAIT = (NB - 2) * A_ISS + NGA + NGB + SUBS * 2 * NPW;
     // One to three K-tiles (wide_kernel's short path): everything is loaded up front, K-tile by
     // K-tile its chunk, scales and B operands; the operations issued after chunk c's copies
     static constexpr int short_wait(int nk, int c) {
-        return NGA + 1 + SUBS * 2 * NPW + (nk - 1 - c) * (A_ISS + NGA + 1 + SUBS * 2 * NPW);
+        return NGA + NGB + SUBS * 2 * NPW + (nk - 1 - c) * (A_ISS + NGA + NGB + SUBS * 2 * NPW);
     }
     // the short path holds a set of B operands per K-tile: up to three K-tiles on the 128 x 256
     // tile, one on 128 x 384; none on 128 x 512 and 256 x 256, whose masked and repacked-A
     // instantiations would then spill (the registers are allocated for the whole kernel)
-    static constexpr int SHORT_MAX = MB == 4 && NPW == 2 ? 3 : MB == 4 && NPW == 3 ? 1 : 0;
+    static constexpr int SHORT_MAX = MB == 4 && NPW == 2 ? (short_wait(3, 0) <= 63 ? 3 : 2)
+                                     : MB == 4 && NPW == 3 ? 1 : 0;
     static_assert(MB == 4 || MB == 8, "128 or 256 rows");
-    static_assert(NPW >= 1 && NPW <= 4, "B scale group holds <= 4 blocks");
+    static_assert(NPW >= 1 && NPW <= 4 && GA <= 4, "a scale group holds <= 4 blocks");
+    static_assert(MB % GA == 0 && NPW % GB == 0, "whole scale groups");
     // NB = 3: the prologue issues chunk 1 before the loop, and the count above then holds for
     // it too (more loads follow chunk 1 in the prologue, the B loads of slabs 1 and 2, than
     // follow a chunk's last copy in the loop)
@@ -130,15 +132,16 @@ struct WideGeom {
     static_assert(short_wait(SHORT_MAX > 0 ? SHORT_MAX : 1, 0) <= 63, "vmcnt range (short path)");
 };
 
-// acc[mi][ni] += A(mi) * B(ni) with the scale bytes mi % 4 of sa and ni of sb (op_sel must be a
+// acc[mi][ni] += A(mi) * B(ni) with the scale bytes mi % GA of sa and ni % GB of sb (op_sel must be a
 // constant: mi and ni are known at compile time wherever this is called from an unrolled loop).
-template <int MB, int NPW>
+template <int MB, int NPW, int GA = 4, int GB = 4>
 __device__ __forceinline__ void wide_mfma(v16f (&acc)[MB][NPW], int mi, int ni, const v8i& a,
                                           const v8i& b, int sa, int sb) {
     switch (mi * 4 + ni) {
 #define WX_CASE(I, J)                                                                   \
     case I * 4 + J:                                                                     \
-        if constexpr (I < MB && J < NPW) acc[I][J] = mfma_fp6<I % 4, J>(acc[I][J], a, b, sa, sb); \
+        if constexpr (I < MB && J < NPW)                                                \
+            acc[I][J] = mfma_fp6<I % GA, J % GB>(acc[I][J], a, b, sa, sb);              \
         break;
 #define WX_ROW(I) WX_CASE(I, 0) WX_CASE(I, 1) WX_CASE(I, 2) WX_CASE(I, 3)
         WX_ROW(0) WX_ROW(1) WX_ROW(2) WX_ROW(3) WX_ROW(4) WX_ROW(5) WX_ROW(6) WX_ROW(7)
@@ -148,16 +151,16 @@ __device__ __forceinline__ void wide_mfma(v16f (&acc)[MB][NPW], int mi, int ni, 
 }
 
 template <int MB_, int NPW_, int NB_, int XG, typename OutT, bool SPLIT, bool ASH, bool MASK,
-          bool STREAM, int ONE = 0, bool SWZ = false>
+          bool STREAM, int ONE = 0, bool SWZ = false, int GA_ = 4, int GB_ = NPW_>
 __global__ void __launch_bounds__(256, 1)
     wide_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ Bsh,
                 const uint8_t* __restrict__ sA, const uint8_t* __restrict__ sB,
                 OutT* __restrict__ D, float* __restrict__ ws, int M, int N, int Kp,
                 int A_row_bytes, int S) {
-    using G = WideGeom<MB_, NPW_, NB_, SWZ>;
+    using G = WideGeom<MB_, NPW_, NB_, SWZ, GA_, GB_>;
     static_assert(!SWZ || (!ASH && !MASK && ONE == 0), "SWZ: row-major A, unmasked tiles");
     constexpr int MT = G::MT, NT = G::NT, MB = G::MB, NPW = G::NPW, NB = G::NB;
-    constexpr int NGA = G::NGA, GA = G::GA, NSET = G::NSET, NMF = G::NMF;
+    constexpr int NGA = G::NGA, GA = G::GA, NGB = G::NGB, GB = G::GB, NSET = G::NSET, NMF = G::NMF;
     constexpr int CHUNK = G::CHUNK;
     __shared__ __attribute__((aligned(1024))) char lds[G::LDS];
 
@@ -226,7 +229,7 @@ __global__ void __launch_bounds__(256, 1)
     // ---- B operand and scale loads of this wave
     const int b_blk_last = (N + 31) / 32 - 1;
     const int sa_grp_last = ((M + 31) / 32 + GA - 1) / GA - 1;
-    const int sb_grp_last = ((N + 31) / 32 + NPW - 1) / NPW - 1;
+    const int sb_grp_last = ((N + 31) / 32 + GB - 1) / GB - 1;
     // The B operand and scale loads are buffer loads: a resource per B block column and per scale
     // group (base address in SGPRs), the lane's part as a constant VGPR offset, the K-tile as a
     // scalar offset and the slab as the instruction's immediate, so a load needs no address
@@ -239,7 +242,7 @@ __global__ void __launch_bounds__(256, 1)
         if (MASK) blk = min(blk, b_blk_last);
         b_rs[ni] = raw_rsrc(opaque_gptr(Bsh + (size_t)blk * k64n * OPBLK_BYTES));
     }
-    // the lane's scale dwords of a K-tile (the dword of slab s at + 4 s), per A group and for B
+    // the lane's scale dwords of a K-tile (the dword of slab s at + 4 s), per A and B group
     rsrc_t sa_rs[NGA];
 #pragma unroll
     for (int g = 0; g < NGA; g++) {
@@ -247,9 +250,13 @@ __global__ void __launch_bounds__(256, 1)
         if (MASK) ga = min(ga, sa_grp_last);
         sa_rs[g] = raw_rsrc(opaque_gptr(sA + (size_t)ga * k_tiles * 64 * 12));
     }
-    int gb = wg_n * G::NWAVES + wave;
-    if (MASK) gb = min(gb, sb_grp_last);
-    const rsrc_t sb_rs = raw_rsrc(opaque_gptr(sB + (size_t)gb * k_tiles * 64 * 12));
+    rsrc_t sb_rs[NGB];
+#pragma unroll
+    for (int g = 0; g < NGB; g++) {
+        int gb = (wg_n * G::NWAVES + wave) * NGB + g;
+        if (MASK) gb = min(gb, sb_grp_last);
+        sb_rs[g] = raw_rsrc(opaque_gptr(sB + (size_t)gb * k_tiles * 64 * 12));
+    }
     const int v_b0 = (int)opaque_v(16 * lane), v_b1 = (int)opaque_v(1024 + 8 * lane);
     const int v_sc = (int)opaque_v(12 * lane);
 
@@ -263,12 +270,14 @@ __global__ void __launch_bounds__(256, 1)
         const v4i y1w = __builtin_shufflevector(y1, y1, 0, 1, -1, -1);
         v = __builtin_shufflevector(y0, y1w, 0, 1, 2, 3, 4, 5, -1, -1);
     };
-    // the lane's three slab scale dwords of K-tile kt, for each A group and for B
-    auto load_scales = [&](v3i (&a)[NGA], v3i& b, int kt) {
+    // the lane's three slab scale dwords of K-tile kt, for each A and B group
+    auto load_scales = [&](v3i (&a)[NGA], v3i (&b)[NGB], int kt) {
 #pragma unroll
         for (int g = 0; g < NGA; g++)
             a[g] = __builtin_bit_cast(v3i, __builtin_amdgcn_raw_buffer_load_b96(sa_rs[g], v_sc, kt * 768, 0));
-        b = __builtin_bit_cast(v3i, __builtin_amdgcn_raw_buffer_load_b96(sb_rs, v_sc, kt * 768, 0));
+#pragma unroll
+        for (int g = 0; g < NGB; g++)
+            b[g] = __builtin_bit_cast(v3i, __builtin_amdgcn_raw_buffer_load_b96(sb_rs[g], v_sc, kt * 768, 0));
     };
 
     // ---- A operand reads (LDS): slab s of the chunk in buffer BUF, block mi. The addresses are
@@ -329,7 +338,7 @@ __global__ void __launch_bounds__(256, 1)
 
     v8i RB[SUBS][NPW];        // B operands, slot s = slab s of a K-tile
     v8i RA[NSET][MB];         // A operands
-    v3i sc_a[2][NGA], sc_b[2];  // scale dwords of K-tiles of even and of odd index
+    v3i sc_a[2][NGA], sc_b[2][NGB];  // scale dwords of K-tiles of even and of odd index
 
     if constexpr (G::SHORT_MAX > 0 || ONE > 0) {
         // One K-tile, or on the 128 x 256 tile up to three (K <= 576, or a split segment that
@@ -341,7 +350,7 @@ __global__ void __launch_bounds__(256, 1)
             constexpr int NK = decltype(nk)::value;
             static_assert(G::short_wait(NK, 0) <= 63, "vmcnt range (short path)");
             v8i RBk[NK][SUBS][NPW];
-            v3i ska[NK][NGA], skb[NK];
+            v3i ska[NK][NGA], skb[NK][NGB];
             static_for<NK>([&](auto cc) {
                 constexpr int c = decltype(cc)::value;
 #pragma unroll
@@ -383,8 +392,9 @@ __global__ void __launch_bounds__(256, 1)
                         const int ni = k / MB, mi = k % MB;
                         const int g = mi / GA;
                         const int sa = s == 0 ? ska[C][g].x : s == 1 ? ska[C][g].y : ska[C][g].z;
-                        const int sb = s == 0 ? skb[C].x : s == 1 ? skb[C].y : skb[C].z;
-                        wide_mfma<MB, NPW>(acc, mi, ni, RA[cur][mi], RBk[C][s][ni], sa, sb);
+                        const v3i cb = skb[C][ni / GB];
+                        const int sb = s == 0 ? cb.x : s == 1 ? cb.y : cb.z;
+                        wide_mfma<MB, NPW, GA, GB>(acc, mi, ni, RA[cur][mi], RBk[C][s][ni], sa, sb);
 #pragma unroll
                         for (int i = 0; i < MB; i++)
                             if (k == G::read_k(i) && (MORE || s + 1 < SUBS)) {
@@ -417,11 +427,13 @@ __global__ void __launch_bounds__(256, 1)
             short_path(std::integral_constant<int, 1>{});
             return;
         }
-        if constexpr (G::SHORT_MAX >= 3) {
+        if constexpr (G::SHORT_MAX >= 2) {
             if (nkt == 2) {
                 short_path(std::integral_constant<int, 2>{});
                 return;
             }
+        }
+        if constexpr (G::SHORT_MAX >= 3) {
             if (nkt == 3) {
                 short_path(std::integral_constant<int, 3>{});
                 return;
@@ -495,8 +507,9 @@ __global__ void __launch_bounds__(256, 1)
                 const int ni = k / MB, mi = k % MB;
                 const int g = mi / GA;
                 const int sa = s == 0 ? sc_a[Q][g].x : s == 1 ? sc_a[Q][g].y : sc_a[Q][g].z;
-                const int sb = s == 0 ? sc_b[Q].x : s == 1 ? sc_b[Q].y : sc_b[Q].z;
-                wide_mfma<MB, NPW>(acc, mi, ni, RA[cur][mi], RB[s][ni], sa, sb);
+                const v3i cb = sc_b[Q][ni / GB];
+                const int sb = s == 0 ? cb.x : s == 1 ? cb.y : cb.z;
+                wide_mfma<MB, NPW, GA, GB>(acc, mi, ni, RA[cur][mi], RB[s][ni], sa, sb);
                 if (s == 0 && k == 0) load_scales(sc_a[1 - Q], sc_b[1 - Q], kt_next);
                 if (ci < G::cps(s) && k == G::copy_k(ci)) {
                     a_copy(c0 + ci, kt_copy, CBufC{});

@@ -459,6 +459,14 @@ int kernel_for(const TileChoice& tc) {
 
 Plan plan_for(int out_type, int M, int N, int Kp, size_t ws_bytes, bool* unsplit);
 
+// The A layout a plan is launched with: a plan that repacks A reads the rows as they are where the
+// launch layer has a faster kernel for them (the plan's workspace is then not touched for A).
+int layout_of(const Plan& pl, int M, int N, int kernel) {
+    return pl.repack && kernel == MXFP6_KERNEL_TILE && !mxfp6_hip_prefers_rows(M, N, pl.S, pl.tc.MT)
+               ? MXFP6_A_REPACK
+               : MXFP6_A_ROWS;
+}
+
 int gemm_checked(int out_type, int M, int N, int Kp, const void* dA, const void* dBsh,
                  const uint8_t* dsA, const uint8_t* dsB, void* dD, int A_row_bytes, void* ws,
                  size_t ws_bytes, void* stream) {
@@ -473,10 +481,9 @@ int gemm_checked(int out_type, int M, int N, int Kp, const void* dA, const void*
                      "got %zu; running unsplit. Size it with gemm_workspace_size().\n",
                      M, N, Kp, splitk_segments(M, N, Kp), workspace_bytes(M, N, Kp), ws_bytes);
     const int kernel = kernel_for(pl.tc);
-    const bool rp = pl.repack && kernel == MXFP6_KERNEL_TILE;
     if (kernel != MXFP6_KERNEL_TILE && (M % 64 != 0 || N % 64 != 0)) return MXFP6_ERR_TILE;
-    return run(out_type, M, N, Kp, pl.tc, pl.S, rp ? MXFP6_A_REPACK : MXFP6_A_ROWS, kernel, dA,
-               dBsh, dsA, dsB, dD, A_row_bytes, ws, stream);
+    return run(out_type, M, N, Kp, pl.tc, pl.S, layout_of(pl, M, N, kernel), kernel, dA, dBsh, dsA,
+               dsB, dD, A_row_bytes, ws, stream);
 }
 
 // The plan gemm() runs for a workspace of ws_bytes: a measured plan of the shape when the
@@ -510,9 +517,10 @@ struct TuneCall {
 
 int tune_launch(void* ctx) {
     const TuneCall& c = *static_cast<const TuneCall*>(ctx);
+    const int kernel = kernel_for(c.plan.tc);
     return run(c.out_type, c.M, c.N, c.Kp, c.plan.tc, c.plan.S,
-               c.plan.repack ? MXFP6_A_REPACK : MXFP6_A_ROWS, kernel_for(c.plan.tc), c.dA, c.dBsh,
-               c.dsA, c.dsB, c.dD, c.A_row_bytes, c.ws, c.stream);
+               layout_of(c.plan, c.M, c.N, kernel), kernel, c.dA, c.dBsh, c.dsA, c.dsB, c.dD,
+               c.A_row_bytes, c.ws, c.stream);
 }
 }  // namespace
 
