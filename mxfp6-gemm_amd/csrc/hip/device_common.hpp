@@ -19,8 +19,6 @@ typedef int v6i_a8 __attribute__((__vector_size__(24), __aligned__(8)));
 // 12 bytes, 4-byte aligned (one ds_read_b96)
 typedef int v3i_a4 __attribute__((__vector_size__(12), __aligned__(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-// 16 bytes, 4-byte aligned (one global_load_dwordx4)
-typedef float v4f_a4 __attribute__((__vector_size__(16), __aligned__(4)));
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef unsigned v6u __attribute__((ext_vector_type(6)));
 
