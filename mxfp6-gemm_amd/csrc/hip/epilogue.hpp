@@ -30,34 +30,65 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[MPW][NPW], OutT* __
             // that the even lane holds rows +0 and +2 of both columns and the odd lane rows +1
             // and +3 (one quad_perm DPP move and three byte permutes per 4 values), halving the
             // store instructions. The conversions are the per-element ones of cvt_out.
+            // A row of one block is 64 bytes, half a cache line, and D at these widths is bound by
+            // how many lines the stores touch: where a wave owns two blocks side by side they are
+            // stored together, 128 contiguous bytes of a row (two of them) an instruction. Against a
+            // block at a time (four half lines an instruction), three operand sets in turn: 8192 x
+            // 8192 x 1024 76.7 -> 71.0 us, 8192 x 8192 x 2048 130 -> 118, 4096 x 4096 x 1024 24.0 ->
+            // 19.3, 8192 x 28672 x 1024 254 -> 220, 8192^3 349 -> 340.
             const bool odd = (lane & 1) != 0;
             const uint32_t sel_send = odd ? 0x05040100u : 0x07060302u;
             const uint32_t sel_a = odd ? 0x03020504u : 0x05040100u;
             const uint32_t sel_b = odd ? 0x03020706u : 0x07060100u;
             const int m_p = m_w + (lane & 1), n_p = n_w & ~1;
+            auto swap_pair = [](uint32_t v) {
+                // quad_perm [1, 0, 3, 2]
+                return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false);
+            };
+            // values 4 g .. 4 g + 3 of a block: rows +0 / +1 (even / odd lane) in oa, +2 / +3 in ob
+            auto rows4 = [&](const v16f& a, int g, uint32_t& oa, uint32_t& ob) {
+                const uint32_t p01 = half_bits(cvt_out<OutT>(a[4 * g])) |
+                                     (half_bits(cvt_out<OutT>(a[4 * g + 1])) << 16);
+                const uint32_t p23 = half_bits(cvt_out<OutT>(a[4 * g + 2])) |
+                                     (half_bits(cvt_out<OutT>(a[4 * g + 3])) << 16);
+                const uint32_t recv = swap_pair(__builtin_amdgcn_perm(p23, p01, sel_send));
+                oa = __builtin_amdgcn_perm(recv, p01, sel_a);
+                ob = __builtin_amdgcn_perm(recv, p23, sel_b);
+            };
+            auto put = [&](int m, int n, uint32_t v) {
+                if (!MASK || m < M) store_out<NT>(reinterpret_cast<uint32_t*>(D + (size_t)m * N + n), v);
+            };
 #pragma unroll
-            for (int mi = 0; mi < MPW; mi++)
+            for (int mi = 0; mi < MPW; mi++) {
 #pragma unroll
-                for (int ni = 0; ni < NPW; ni++)
+                for (int ni = 0; ni + 1 < NPW; ni += 2)
 #pragma unroll
                     for (int g = 0; g < 4; g++) {
-                        const v16f& a = acc[mi][ni];
-                        const uint32_t p01 = half_bits(cvt_out<OutT>(a[4 * g])) |
-                                             (half_bits(cvt_out<OutT>(a[4 * g + 1])) << 16);
-                        const uint32_t p23 = half_bits(cvt_out<OutT>(a[4 * g + 2])) |
-                                             (half_bits(cvt_out<OutT>(a[4 * g + 3])) << 16);
-                        const uint32_t send = __builtin_amdgcn_perm(p23, p01, sel_send);
-                        const uint32_t recv = (uint32_t)__builtin_amdgcn_mov_dpp(
-                            (int)send, 0xB1, 0xF, 0xF, false);  // quad_perm [1, 0, 3, 2]
-                        const uint32_t oa = __builtin_amdgcn_perm(recv, p01, sel_a);
-                        const uint32_t ob = __builtin_amdgcn_perm(recv, p23, sel_b);
-                        const int m = m_p + mi * 32 + 8 * g, n = n_p + ni * 32;
+                        // the pair trades again: the even lane holds all four rows of block ni, the
+                        // odd lane those of block ni + 1
+                        uint32_t a0, b0, a1, b1;
+                        rows4(acc[mi][ni], g, a0, b0);
+                        rows4(acc[mi][ni + 1], g, a1, b1);
+                        const uint32_t ra = swap_pair(odd ? a0 : a1), rb = swap_pair(odd ? b0 : b1);
+                        const int m = m_w + mi * 32 + 8 * g, n = n_p + (ni + (lane & 1)) * 32;
                         if (MASK && n >= N) continue;  // n even and N even: n + 1 < N as well
-                        uint32_t* d0 = reinterpret_cast<uint32_t*>(D + (size_t)m * N + n);
-                        if (!MASK || m < M) store_out<NT>(d0, oa);
-                        if (!MASK || m + 2 < M)
-                            store_out<NT>(reinterpret_cast<uint32_t*>(D + (size_t)(m + 2) * N + n), ob);
+                        put(m, n, odd ? ra : a0);
+                        put(m + 1, n, odd ? a1 : ra);
+                        put(m + 2, n, odd ? rb : b0);
+                        put(m + 3, n, odd ? b1 : rb);
                     }
+                if constexpr (NPW % 2 != 0) {
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        uint32_t oa, ob;
+                        rows4(acc[mi][NPW - 1], g, oa, ob);
+                        const int m = m_p + mi * 32 + 8 * g, n = n_p + (NPW - 1) * 32;
+                        if (MASK && n >= N) continue;
+                        put(m, n, oa);
+                        put(m + 2, n, ob);
+                    }
+                }
+            }
             return;
         }
     }
