@@ -412,7 +412,8 @@ bool streams_output(int out_type, int M, int N, int Kp, const TileChoice& tc, in
     const double out = (double)M * N * (out_type == 0 ? 4 : 2);  // FP32 or a 16-bit type
     if (in > LLC_BYTES) return false;
     return in + out > STREAM_FOOTPRINT_BYTES ||
-           (in + out > LLC_BYTES / 2 && out >= STREAM_D_RATIO * in);
+           (in + out > LLC_BYTES / 2 &&
+            out >= (in + out <= STREAM_MID_BYTES ? STREAM_MID_RATIO : STREAM_D_RATIO) * in);
 }
 
 // ws: the workspace of the plan (S, a_layout): split partials first, then (MXFP6_A_REPACK) the

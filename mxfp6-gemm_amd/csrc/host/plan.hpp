@@ -27,24 +27,28 @@ constexpr double A_ROWS_COST = 0.572519;    // extra copy cost per byte of a row
 constexpr double A_ROWS_COST_WIDE = 0.0675946;  // the same for the wide tiles' K-tile chunks
 constexpr double A_ROWS_LONG = 0.158036;    // more per doubling of Kp past 8192 (row-major A)
 constexpr double PLAN_MIN_GAIN = 0.01;     // lead a more complex plan needs over a simpler one
-// An unsplit plan on a wide tile writes D with nontemporal stores when the bytes it reads (operands, scales, the
-// repacked A) fit in MI355X's 256 MiB last-level cache (Infinity Cache) but those and D together
-// exceed STREAM_FOOTPRINT_BYTES: D then no longer evicts the operands the tiles re-read. Measured:
-// streaming D 6-22% faster above the footprint (8192x16384x2048, 4096x51200x1024,
-// 16384x16384x4096, 1024x102272x2048, 2048x102272x1024), plain stores 5-12% faster below it
-// (8192x8192x2048, 8192x12288x2048, 2048x51200x1024), no difference once the operands alone
-// exceed the cache (2048x102272x4096).
-// Below that footprint, from half the cache on, it does so where D is at least
-// STREAM_D_RATIO times what it reads (short K, many tile rows). Two such calls in a row, on operands
-// and outputs of their own as a program's layers are, then no longer fit the cache together, and the
-// plain stores of one wait for the other's to be written back. Three sets in turn, plain -> streamed:
-// 8192x8192x1024 (D 10x the operands) 100.7 -> 82.4 us, 16384x8192x512 155.8 -> 117.5,
-// 4096x16384x768 79.3 -> 68.0, 16384x4096x512 76.7 -> 72.9; the same set over and over 83.0 -> 84.6,
-// 130.6 -> 116.1, 78.8 -> 67.3, 97.6 -> 65.0. Below half the cache no gain (8192x7168x1024 81.6 ->
-// 80.3, 8192x6144x1024 61.5 -> 68.5), nor at lower ratios where the operands weigh more
-// (2048x28672x1024, 4x: 81.9 -> 85.7; the same set 8192x8192x2048, 5x: 111.0 -> 115.1).
+// An unsplit plan on a wide tile writes D with nontemporal stores by what it reads (operands, scales, the
+// repacked A: "in", at most MI355X's 256 MiB last-level cache) and writes ("out"):
+//   in + out > STREAM_FOOTPRINT_BYTES: D no longer evicts the operands the tiles re-read (6-22% faster,
+//   8192x16384x2048, 4096x51200x1024, 16384x16384x4096, 1024x102272x2048, 2048x102272x1024; no
+//   difference once the operands alone exceed the cache, 2048x102272x4096);
+//   in + out from half the cache to STREAM_MID_BYTES, D no less than STREAM_MID_RATIO of in: two such
+//   calls in a row, on operands and outputs of their own as a program's layers are, no longer fit the
+//   cache together, and the plain stores of one wait for the other's D to be written back. Plain ->
+//   streamed with the epilogue's full-line stores, three sets in turn (the same set over and over):
+//   8192x8192x2048 120.5 -> 103.6 us (109.4 -> 103.5), 8192x8192x4096 198.8 -> 166.9 (167.7 -> 167.4),
+//   4096x14336x4096 188.4 -> 154.5 (156.4 -> 154.1), 8192x5120x8192 243.7 -> 202.1 (203.2 -> 201.4),
+//   1024x28672x4096 98.8 -> 97.2 (78.8 -> 77.3), FP32 4096x6144x4096 90.4 -> 75.6 (73.8 -> 74.8) and
+//   4096x8192x2048 74.0 -> 70.9 (68.1 -> 71.0); 16-bit outputs: 16 of 16 shapes not slower either
+//   way. The gain ends at 240 MB (8192^3 340.8 -> 326.7, 300.3 -> 298.3), below half the cache
+//   it is -2 to 4% (4096x8192x2048 53.2 -> 54.5, 8192x6144x1024 60.5 -> 58.1). The ratio keeps
+//   out the plans that run as 128-row bands (stream_kernel.hpp), whose D is small;
+//   past that up to STREAM_FOOTPRINT_BYTES, D at least STREAM_D_RATIO times in (short K):
+//   16384x8192x512 155.8 -> 117.5 us (130.6 -> 116.1).
 constexpr double LLC_BYTES = 268435456.0;
 constexpr double STREAM_FOOTPRINT_BYTES = 280e6;
+constexpr double STREAM_MID_BYTES = 236e6;
+constexpr double STREAM_MID_RATIO = 0.4;
 constexpr double STREAM_D_RATIO = 8.0;
 
 TileChoice route(int M, int N, int Kp);

@@ -1,6 +1,6 @@
-"""Unsplit plans on wide tiles whose operands and D fill half the 256 MiB last-level cache or more with
-a D of at least 8 times the operands (short K) write D with nontemporal stores: the rule's edges, and
-the values against the direct kernel bit for bit."""
+"""Unsplit plans on wide tiles whose operands and D fill half the 256 MiB last-level cache or more write
+D with nontemporal stores where D is at least 0.4 times the operands (up to 236 MB in all) or 8 times
+(above): the rule's edges, and the values against the direct kernel bit for bit."""
 import pytest
 
 import checks
@@ -11,10 +11,14 @@ import mxfp6_amd as mx
     (8192, 8192, 1024, mx.OUT_BF16, True),    # D 134 MB, 10x the operands
     (8192, 7936, 960, mx.OUT_BF16, True),     # 130 + 12 MB: over half the cache
     (8192, 7168, 1024, mx.OUT_BF16, False),   # 131 MB in all: under it
-    (8192, 8192, 1536, mx.OUT_BF16, False),   # D 7x the operands
-    (4096, 10240, 1024, mx.OUT_F32, True),    # 16-bit D would not fill it
+    (8192, 8192, 4096, mx.OUT_BF16, True),    # D 2.5x, 187 MB in all
+    (8192, 4096, 8192, mx.OUT_BF16, True),    # D 0.85x, 146 MB
+    (256, 18432, 12288, mx.OUT_F32, False),   # D a tenth of the operands
+    (8192, 12288, 3072, mx.OUT_BF16, False),  # 251 MB in all, D 4x
+    (8192, 15360, 512, mx.OUT_BF16, True),    # 262 MB, D over 8x
+    (4096, 10240, 1024, mx.OUT_F32, True),    # 16-bit D would not fill half the cache
     (4096, 10240, 1024, mx.OUT_F16, False),
-    (2048, 28672, 1024, mx.OUT_F16, False)])  # D 4x the operands
+    (2048, 28672, 1024, mx.OUT_F16, True)])
 def test_rule(M, N, K, out_type, want):
     Kp = mx.kpad(K)
     assert mx.splitk_segments(M, N, Kp) == 1
@@ -22,7 +26,7 @@ def test_rule(M, N, K, out_type, want):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,out_type", [(8192, 8192, 1024, mx.OUT_BF16),
+@pytest.mark.parametrize("M,N,K,out_type", [(8192, 8192, 1024, mx.OUT_BF16), (2048, 28672, 1344, mx.OUT_F16),
                                             (4096, 10240, 960, mx.OUT_F32)])
 def test_equals_direct_kernel(M, N, K, out_type):
     from gpu_util import DevProblem, run_direct, run_routed
