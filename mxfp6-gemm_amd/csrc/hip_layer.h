@@ -46,7 +46,7 @@ typedef struct mxfp6_launch_desc {
                           (wide tiles that divide M x N, plain stores; explicit plans only) */
     void* Ash;         /* MXFP6_A_REPACK: M * packed(Kp) bytes */
     int out_stream;    /* 1: the wide tile kernel writes D with nontemporal stores (unsplit plans
-                          whose D would evict the operands from the last-level cache) */
+                          with a large D: the rule and its figures are in csrc/host/plan.hpp) */
     void* stream;      /* hipStream_t */
 } mxfp6_launch_desc;
 
