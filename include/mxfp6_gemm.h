@@ -191,6 +191,22 @@ int mxfp6_gemm_plan(int out_type, int M, int N, int Kp, size_t ws_bytes, int til
  * same either way. */
 int mxfp6_gemm_streams_output(int out_type, int M, int N, int Kp, int A_row_bytes);
 
+/* Kernels a plan's tile runs on (mxfp6_plan_kernel); all give the same bits. */
+typedef enum mxfp6_tile_kernel {
+    MXFP6_TILE_TINY = 0,   /* 32 x 32 tile, K split over a workgroup's waves */
+    MXFP6_TILE_SLAB = 1,   /* A and B staged in LDS, a 64-wide K slab at a time */
+    MXFP6_TILE_WIDE = 2,   /* four waves side by side, B into registers, A staged a K-tile at a time */
+    MXFP6_TILE_STREAM = 3, /* 32- or 64-row tile: B into registers, A staged by a wave of its own */
+    MXFP6_TILE_BAND = 4    /* the same on 128 rows, a 32-column block a wave (small grids) */
+} mxfp6_tile_kernel;
+
+/* The kernel that the plan (tile, splits, a_layout as in mxfp6_gemm_explicit) runs on, a
+ * mxfp6_tile_kernel, or -1 where the plan is not valid. *waves (may be NULL): the computing waves of a
+ * workgroup for STREAM and BAND, else 0; *b_nontemporal (may be NULL): 1 where those load B past the
+ * caches. For tests and benchmarks that name what ran. No counterpart in the reference. */
+int mxfp6_plan_kernel(int out_type, int M, int N, int Kp, const int tile[4], int splits, int a_layout,
+                      int A_row_bytes, int* waves, int* b_nontemporal);
+
 /* Workspace bytes of an explicit plan (0 when splits == 1 and a_repack == 0). */
 size_t mxfp6_plan_workspace_size(int M, int N, int Kp, int splits, int a_repack);
 

@@ -165,7 +165,9 @@ extern "C" int mxfp6_hip_has_tile(int MT, int NT, int mpw, int npw) {
 }
 
 extern "C" int mxfp6_hip_prefers_rows(int M, int N, int splits, int MT) {
-    return MT <= 64 && skinny_runs_wide(M, N, splits, true) ? 1 : 0;
+    const int reported = mxfp6_hip_device_cus();
+    const long cus = reported > 0 ? reported : 256;
+    return MT <= 64 && 5L * ((M + 127) / 128) * ((N + 255) / 256) * splits >= 2 * cus ? 1 : 0;
 }
 
 // Rows of the tiled scale layout: dim rounded up to whole groups of 32 * group rows.

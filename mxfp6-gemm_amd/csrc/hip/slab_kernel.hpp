@@ -404,7 +404,7 @@ hipError_t wide_launch_st(const mxfp6_launch_desc* d, const uint8_t* A, hipStrea
 }
 
 template <int MB, int NPW, int XG, typename KT, bool SPLIT>
-int wide_launch_t(const mxfp6_launch_desc* d, hipStream_t st) {
+int wide_launch_t(const mxfp6_launch_desc* d, const mxfp6_dispatch::TileRun& run, hipStream_t st) {
     using G = WideGeom<MB, NPW, WIDE_NB>;
     static_assert(G::LDS <= 160 * 1024 && WideGeom<MB, NPW, WIDE_NB, true>::LDS <= 160 * 1024,
                   "LDS budget");
@@ -412,7 +412,7 @@ int wide_launch_t(const mxfp6_launch_desc* d, hipStream_t st) {
     // the swizzled staging of row-major A: unmasked tiles, plain stores
     if (d->a_layout == MXFP6_A_ROWS_SWIZZLED && (mask || d->out_stream)) return 2;
     // a grid that leaves many CUs idle runs as 128-row bands of the stream kernel
-    if (const int wn = band_waves(d)) return band_launch<KT, SPLIT>(d, wn, st);
+    if (run.kernel == MXFP6_TILE_BAND) return band_launch<KT, SPLIT>(d, run, st);
     const uint8_t* A = static_cast<const uint8_t*>(d->A);
     if (d->a_layout == MXFP6_A_REPACK) {
         if (repack_rows_launch(A, d->A_row_bytes, d->M, d->Kp / 64, static_cast<uint8_t*>(d->Ash),
@@ -434,9 +434,9 @@ int wide_launch_t(const mxfp6_launch_desc* d, hipStream_t st) {
 // tile's scale groups; A repacked or preshuffled on the slab kernel with one wave row and four wave
 // columns. All give the same bits.
 template <int MT, int NT, typename KT, bool SPLIT>
-int skinny_launch(const mxfp6_launch_desc* d, hipStream_t st) {
-    if (d->a_layout != MXFP6_A_ROWS) return slab_launch_t<MT, NT, 1, 4, 4, 8, KT, SPLIT, false>(d, st);
-    if (skinny_runs_wide(d->M, d->N, d->splits, false)) {
+int skinny_launch(const mxfp6_launch_desc* d, const mxfp6_dispatch::TileRun& run, hipStream_t st) {
+    if (run.kernel == MXFP6_TILE_SLAB) return slab_launch_t<MT, NT, 1, 4, 4, 8, KT, SPLIT, false>(d, st);
+    if (run.kernel == MXFP6_TILE_WIDE) {
         using G = WideGeom<4, 2, WIDE_NB, false, MT / 32, NT / 128>;
         const dim3 grid((unsigned)((d->M + G::MT - 1) / G::MT), (unsigned)((d->N + G::NT - 1) / G::NT),
                         (unsigned)d->splits);
@@ -449,7 +449,7 @@ int skinny_launch(const mxfp6_launch_desc* d, hipStream_t st) {
                    ? 0
                    : 2;
     }
-    return stream_launch<MT / 32, NT / 128, KT, SPLIT>(d, st);
+    return stream_launch<MT / 32, NT / 128, KT, SPLIT>(d, run, st);
 }
 
 // Tile dispatch (declared in slab_run.hpp; instantiated once per (KT, SPLIT) in its own
@@ -457,16 +457,17 @@ int skinny_launch(const mxfp6_launch_desc* d, hipStream_t st) {
 template <typename KT, bool SPLIT>
 int slab_run(const mxfp6_launch_desc* d, hipStream_t st) {
     if (!tile_supported(d->MT, d->NT, d->mpw, d->npw)) return 1;
+    const mxfp6_dispatch::TileRun run = mxfp6_dispatch::tile_run(*d, mxfp6_hip_device_cus());
     // wide tiles: four waves side by side (TileChoice MPW 4 = the A scale group)
-    if (d->MT == 128 && d->NT == 512) return wide_launch_t<4, 4, 8, KT, SPLIT>(d, st);
-    if (d->MT == 128 && d->NT == 256 && d->mpw == 4) return wide_launch_t<4, 2, 8, KT, SPLIT>(d, st);
-    if (d->MT == 256 && d->NT == 256 && d->npw == 2) return wide_launch_t<8, 2, 4, KT, SPLIT>(d, st);
-    if (d->MT == 128 && d->NT == 384) return wide_launch_t<4, 3, 8, KT, SPLIT>(d, st);
+    if (d->MT == 128 && d->NT == 512) return wide_launch_t<4, 4, 8, KT, SPLIT>(d, run, st);
+    if (d->MT == 128 && d->NT == 256 && d->mpw == 4) return wide_launch_t<4, 2, 8, KT, SPLIT>(d, run, st);
+    if (d->MT == 256 && d->NT == 256 && d->npw == 2) return wide_launch_t<8, 2, 4, KT, SPLIT>(d, run, st);
+    if (d->MT == 128 && d->NT == 384) return wide_launch_t<4, 3, 8, KT, SPLIT>(d, run, st);
     // skinny tiles: the stream kernel on row-major A, here preshuffled A (a deeper ring)
-    if (d->MT == 32 && d->NT == 128) return skinny_launch<32, 128, KT, SPLIT>(d, st);
-    if (d->MT == 32 && d->NT == 256) return skinny_launch<32, 256, KT, SPLIT>(d, st);
-    if (d->MT == 64 && d->NT == 128) return skinny_launch<64, 128, KT, SPLIT>(d, st);
-    if (d->MT == 64 && d->NT == 256) return skinny_launch<64, 256, KT, SPLIT>(d, st);
+    if (d->MT == 32 && d->NT == 128) return skinny_launch<32, 128, KT, SPLIT>(d, run, st);
+    if (d->MT == 32 && d->NT == 256) return skinny_launch<32, 256, KT, SPLIT>(d, run, st);
+    if (d->MT == 64 && d->NT == 128) return skinny_launch<64, 128, KT, SPLIT>(d, run, st);
+    if (d->MT == 64 && d->NT == 256) return skinny_launch<64, 256, KT, SPLIT>(d, run, st);
     if (d->MT == 128 && d->NT == 128) return slab_launch_t<128, 128, 2, 2, 4, 6, KT, SPLIT>(d, st);
     if (d->MT == 128 && d->NT == 256) return slab_launch_t<128, 256, 2, 2, 4, 8, KT, SPLIT>(d, st);
     if (d->MT == 256 && d->NT == 192) return slab_launch_t<256, 192, 2, 2, 4, 6, KT, SPLIT>(d, st);

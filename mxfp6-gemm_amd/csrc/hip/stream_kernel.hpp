@@ -22,7 +22,7 @@
 // the Infinity Cache, the same with 2, 4 or 6 K-tiles of loads ahead. So lead past two K-tiles is
 // worth nothing; the lines of A, the padded scale dwords and the number of CUs in use are what
 // counts. That is why A comes in two K-tiles per row piece, only one wave loads A's scales, and WN
-// shrinks when the grid is small (stream_launch). 64 x 28672 x 8192 (three operand sets in turn,
+// shrinks when the grid is small (tile_dispatch.hpp). 64 x 28672 x 8192 (three operand sets in turn,
 // B from HBM): 52.1 us on the slab kernel (B and A through LDS a slab at a time, every wave
 // copying), 38.2 here: 5.0 TB/s of operands; without A's copies and scales 30.5.
 // NT: B's loads are nontemporal where B exceeds half the last-level cache and is read by one tile
@@ -40,7 +40,7 @@
 // that exists; stores are masked.
 #pragma once
 
-#include "../hip_layer.h"
+#include "../tile_dispatch.hpp"
 #include "device_common.hpp"
 #include "epilogue.hpp"
 #include "lds_dma.hpp"
@@ -322,16 +322,8 @@ __global__ void __launch_bounds__(64 * (WN_ == 0 ? 7 : WN_ + 1), 1)
                                            (wg_n * WN + wave) * NPW * 32 + (le & 31), le, wg_z);
 }
 
-// One launch for a tile of grouping (MB, NPW), four computing waves wide as the router counts it.
-// The K-segment partials go to d->ws when SPLIT. Fewer computing waves a workgroup where four
-// would leave CUs idle or load them unevenly (three operand sets in turn, 177 shapes with up to
-// 4,500 workgroups; the slab kernel was 1.02-1.63x slower on every one of them):
-//   one 32-column block a wave (NPW 1): two waves below 3/5 of the CUs, and on 32 rows one
-//   where two stay below that as well (32 x 384 x 12928 in 16 segments, 48 workgroups of four:
-//   four 1.13x, two 1.04x, one 1; 16 x 1024 x 10880, 128: four 1.11x, two 1);
-//   two blocks a wave: two waves on more workgroups than CUs, which four waves' registers run
-//   one round at a time (96 x 23552 x 2112, 276 workgroups: four 1.25x two; 2240 x 2176 x 576,
-//   315: 1.21x; on 144-256 workgroups four are 0-12% faster).
+// One launch for a tile of grouping (MB, NPW) with WN computing waves a workgroup. The K-segment
+// partials go to d->ws when SPLIT.
 template <int MB, int NPW, int WN, typename KT, bool SPLIT>
 hipError_t stream_launch_w(const mxfp6_launch_desc* d, bool ntb, hipStream_t st) {
     using G = StreamGeom<MB, NPW, WN>;
@@ -351,66 +343,29 @@ hipError_t stream_launch_w(const mxfp6_launch_desc* d, bool ntb, hipStream_t st)
                          d->N, d->Kp, d->A_row_bytes, SPLIT ? d->splits : 1, NPW);
 }
 
-// Returns 0, or 2 when the launch fails.
+// run.waves computing waves (tile_dispatch.hpp). Returns 0, or 2 when the launch fails.
 template <int MB, int NPW, typename KT, bool SPLIT>
-int stream_launch(const mxfp6_launch_desc* d, hipStream_t st) {
-    const int reported = mxfp6_hip_device_cus();
-    const long cus = reported > 0 ? reported : 256;
-    auto wgs = [&](int wn) {
-        return (long)((d->M + 32 * MB - 1) / (32 * MB)) * ((d->N + 32 * NPW * wn - 1) / (32 * NPW * wn)) *
-               d->splits;
-    };
-    // B read once (one tile row) and more than half of the 256 MiB last-level cache
-    const bool ntb = d->M <= 32 * MB && (double)d->N * (d->Kp / 4 * 3) > 128.0 * (1 << 20);
+int stream_launch(const mxfp6_launch_desc* d, const mxfp6_dispatch::TileRun& run, hipStream_t st) {
     hipError_t e;
-    if constexpr (NPW == 1) {
-        if (MB == 1 && 5 * wgs(2) < 3 * cus)
-            e = stream_launch_w<MB, NPW, MB == 1 ? 1 : 2, KT, SPLIT>(d, ntb, st);
-        else if (5 * wgs(4) < 3 * cus)
-            e = stream_launch_w<MB, NPW, 2, KT, SPLIT>(d, ntb, st);
-        else
-            e = stream_launch_w<MB, NPW, 4, KT, SPLIT>(d, ntb, st);
-    } else {
-        if (wgs(4) > cus && !ntb)
-            e = stream_launch_w<MB, NPW, 2, KT, SPLIT>(d, ntb, st);
-        else
-            e = stream_launch_w<MB, NPW, 4, KT, SPLIT>(d, ntb, st);
-    }
+    if (run.waves == 4)
+        e = stream_launch_w<MB, NPW, 4, KT, SPLIT>(d, run.nt_b, st);
+    else if (MB == 1 && NPW == 1 && run.waves == 1)
+        e = stream_launch_w<MB, NPW, MB == 1 && NPW == 1 ? 1 : 2, KT, SPLIT>(d, run.nt_b, st);
+    else
+        e = stream_launch_w<MB, NPW, 2, KT, SPLIT>(d, run.nt_b, st);
     return e == hipSuccess ? 0 : 2;
 }
 
-// Computing waves of the BAND launch that runs a wide tile's plan on row-major A, or 0 where the wide
-// kernel is the better one: the fewest with which the plan's workgroups run in one round of the
-// CUs. Up to four were never slower than the wide kernel on 43 measured shapes, three operand sets in
-// turn (three waves 2048 x 1152 x 2128 1.25x, 128 x 24576 x 4096 1.52x; four 512 x 8192 x 2048 1.00x,
-// 1203 x 2560 x 1408 1.12x, 128 x 2048 x 50116 in 16 segments 1.16x); five only where B is no small
-// part of the 256 MiB last-level cache (57 MB 1.03-1.08x unsplit, 0.90 split; 75 MB 1.29x, 126 MB
-// in two segments 1.18x, 170 MB 1.32x; 28 MB 0.91, 42 MB 1.00), for there the wide kernel's loads, one
-// K-tile ahead, wait on HBM; six lost but for one shape (682 x 1280 x 27520 in 6 segments 0.76, 256 x
-// 7040 x 9920 in 3 0.89; 128 x 6016 x 18944 in 8 1.15x). Segments of fewer than eight K-tiles keep the
-// wide kernel, which has short paths for them.
-inline int band_waves(const mxfp6_launch_desc* d) {
-    if (d->a_layout != MXFP6_A_ROWS || d->mpw != 4 || d->out_stream || d->Kp / 192 < 8 * d->splits)
-        return 0;
-    const int reported = mxfp6_hip_device_cus();
-    const long cus = reported > 0 ? reported : 256;
-    const long rows = (long)((d->M + 127) / 128) * d->splits, blks = (d->N + 31) / 32;
-    const bool large_b = (double)d->N * (d->Kp / 4 * 3) > 64.0 * (1 << 20);
-    for (int wn = 2; wn <= (large_b ? 5 : 4); wn++)
-        if (rows * ((blks + wn - 1) / wn) <= cus) return wn;
-    return 0;
-}
-
-// Returns 0, or 2 when the launch fails.
+// BAND with run.waves computing waves. Returns 0, or 2 when the launch fails.
 template <typename KT, bool SPLIT>
-int band_launch(const mxfp6_launch_desc* d, int wn, hipStream_t st) {
+int band_launch(const mxfp6_launch_desc* d, const mxfp6_dispatch::TileRun& run, hipStream_t st) {
     using G = StreamGeom<4, 1, 0>;
-    const bool ntb = d->M <= 128 && (double)d->N * (d->Kp / 4 * 3) > 128.0 * (1 << 20);
+    const int wn = run.waves;
     const dim3 grid((unsigned)((d->M + 127) / 128), (unsigned)((d->N + 32 * wn - 1) / (32 * wn)),
                     (unsigned)d->splits);
     const hipError_t e = launch_kernel(
-        ntb ? stream_kernel<4, 1, 0, 4, KT, SPLIT, true, true>
-            : stream_kernel<4, 1, 0, 4, KT, SPLIT, true, false>,
+        run.nt_b ? stream_kernel<4, 1, 0, 4, KT, SPLIT, true, true>
+                 : stream_kernel<4, 1, 0, 4, KT, SPLIT, true, false>,
         grid, dim3(64 * (wn + G::NCW)), st, static_cast<const uint8_t*>(d->A),
         static_cast<const uint8_t*>(d->Bsh), d->sA, d->sB, SPLIT ? nullptr : static_cast<KT*>(d->D),
         SPLIT ? d->ws : nullptr, d->M, d->N, d->Kp, d->A_row_bytes, SPLIT ? d->splits : 1, d->npw);

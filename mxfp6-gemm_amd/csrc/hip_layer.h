@@ -67,7 +67,7 @@ void* mxfp6_hip_scratch(size_t* bytes);
 int mxfp6_hip_clock_sample(uint64_t* out, int nwg, void* stream);
 
 /* 1 when a plan on this tile that repacks A first runs faster on row-major A (the skinny tiles on
- * enough workgroups, slab_run.hpp skinny_runs_wide), else 0. The output bits are the same. */
+ * enough workgroups), else 0. The output bits are the same. */
 int mxfp6_hip_prefers_rows(int M, int N, int splits, int MT);
 
 /* Compute units of the current HIP device (hipDeviceAttributeMultiprocessorCount, read once per

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "../hip_layer.h"
+#include "../tile_dispatch.hpp"
 #include "mxfp6/gemm.hpp"
 #include "mxfp6_gemm.h"
 #include "plan.hpp"
@@ -416,12 +417,10 @@ bool streams_output(int out_type, int M, int N, int Kp, const TileChoice& tc, in
             out >= (in + out <= STREAM_MID_BYTES ? STREAM_MID_RATIO : STREAM_D_RATIO) * in);
 }
 
-// ws: the workspace of the plan (S, a_layout): split partials first, then (MXFP6_A_REPACK) the
-// repacked A at the next 256-byte boundary.
-int run(int out_type, int M, int N, int Kp, const TileChoice& tc, int S, int a_layout, int kernel,
-        const void* dA, const void* dBsh, const uint8_t* dsA, const uint8_t* dsB, void* dD,
-        int A_row_bytes, void* ws, void* stream) {
-    mxfp6_launch_desc d;
+// The launch descriptor of a plan, without its pointers.
+mxfp6_launch_desc describe(int out_type, int M, int N, int Kp, const TileChoice& tc, int S, int a_layout,
+                           int kernel, int A_row_bytes) {
+    mxfp6_launch_desc d = {};
     d.kernel = kernel;
     d.out_type = out_type;
     d.M = M;
@@ -433,21 +432,30 @@ int run(int out_type, int M, int N, int Kp, const TileChoice& tc, int S, int a_l
     d.npw = tc.NPW;
     d.splits = S;
     d.A_row_bytes = A_row_bytes;
+    d.a_layout = a_layout;
+    d.out_stream = kernel == MXFP6_KERNEL_TILE && a_layout != MXFP6_A_ROWS_SWIZZLED &&
+                           streams_output(out_type, M, N, Kp, tc, S, a_layout == MXFP6_A_REPACK,
+                                          A_row_bytes)
+                       ? 1
+                       : 0;
+    return d;
+}
+
+// ws: the workspace of the plan (S, a_layout): split partials first, then (MXFP6_A_REPACK) the
+// repacked A at the next 256-byte boundary.
+int run(int out_type, int M, int N, int Kp, const TileChoice& tc, int S, int a_layout, int kernel,
+        const void* dA, const void* dBsh, const uint8_t* dsA, const uint8_t* dsB, void* dD,
+        int A_row_bytes, void* ws, void* stream) {
+    mxfp6_launch_desc d = describe(out_type, M, N, Kp, tc, S, a_layout, kernel, A_row_bytes);
     d.A = dA;
     d.Bsh = dBsh;
     d.sA = dsA;
     d.sB = dsB;
     d.D = dD;
     d.ws = S > 1 ? static_cast<float*>(ws) : nullptr;
-    d.a_layout = a_layout;
     d.Ash = a_layout == MXFP6_A_REPACK
                 ? static_cast<uint8_t*>(ws) + (split_bytes(M, N, S) + 255) / 256 * 256
                 : nullptr;
-    d.out_stream = kernel == MXFP6_KERNEL_TILE && a_layout != MXFP6_A_ROWS_SWIZZLED &&
-                           streams_output(out_type, M, N, Kp, tc, S, a_layout == MXFP6_A_REPACK,
-                                          A_row_bytes)
-                       ? 1
-                       : 0;
     d.stream = stream;
     const int rc = mxfp6_hip_launch(&d);
     return rc == 0 ? MXFP6_OK : rc == 1 ? MXFP6_ERR_TILE : MXFP6_ERR_HIP;
@@ -902,6 +910,21 @@ extern "C" int mxfp6_gemm_plan(int out_type, int M, int N, int Kp, size_t ws_byt
         return MXFP6_ERR_ARG;
     if (tile == nullptr || splits == nullptr || a_repack == nullptr) return MXFP6_ERR_NULL;
     return plan::plan_info(out_type, M, N, Kp, ws_bytes, tile, splits, a_repack);
+}
+
+extern "C" int mxfp6_plan_kernel(int out_type, int M, int N, int Kp, const int tile[4], int splits,
+                                 int a_layout, int A_row_bytes, int* waves, int* b_nontemporal) {
+    if (out_type < 0 || out_type > 2 || M <= 0 || N <= 0 || Kp <= 0 || Kp % K_TILE != 0 ||
+        tile == nullptr || splits < 1 || splits > Kp / K_TILE || a_layout < MXFP6_A_ROWS ||
+        a_layout > MXFP6_A_ROWS_SWIZZLED || !mxfp6_hip_has_tile(tile[0], tile[1], tile[2], tile[3]))
+        return -1;
+    const mxfp6_launch_desc d =
+        plan::describe(out_type, M, N, Kp, {tile[0], tile[1], tile[2], tile[3]}, splits, a_layout,
+                       MXFP6_KERNEL_TILE, A_row_bytes);
+    const mxfp6_dispatch::TileRun r = mxfp6_dispatch::tile_run(d, mxfp6_hip_device_cus());
+    if (waves != nullptr) *waves = r.waves;
+    if (b_nontemporal != nullptr) *b_nontemporal = r.nt_b ? 1 : 0;
+    return r.kernel;
 }
 
 extern "C" size_t mxfp6_plan_workspace_size(int M, int N, int Kp, int splits, int a_repack) {

@@ -67,6 +67,8 @@ SIGNATURES = {
     "mxfp6_gemm_tune_load": (C.c_int, [C.c_char_p, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "mxfp6_gemm_plan": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.c_size_t,
                                   C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int)]),
+    "mxfp6_plan_kernel": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int), C.c_int,
+                                    C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "mxfp6_plan_workspace_size": (C.c_size_t, [C.c_int, C.c_int, C.c_int, C.c_int, C.c_int]),
     "mxfp6_preshuffle_rows_async": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, _vp, _vp]),
     "mxfp6_quantize_async": (C.c_int, [_vp, C.c_int, C.c_int, _vp, C.c_size_t, _vp, C.c_int, _vp]),
@@ -268,6 +270,21 @@ def gemm_plan(out_type, M, N, Kp, ws_bytes):
 def streams_output(out_type, M, N, Kp, A_row_bytes):
     """Whether gemm()'s plan writes D with nontemporal stores for this call."""
     return bool(lib().mxfp6_gemm_streams_output(out_type, M, N, Kp, A_row_bytes))
+
+
+TILE_KERNELS = ("tiny", "slab", "wide", "stream", "band")  # mxfp6_tile_kernel
+
+
+def plan_kernel(out_type, M, N, Kp, tile, splits=1, a_layout=A_ROWS, A_row_bytes=None):
+    """(kernel, waves, b_nontemporal) that a plan runs on: one of TILE_KERNELS, the computing waves of a
+    stream or band workgroup (else 0) and whether those load B past the caches."""
+    w, nt = C.c_int(0), C.c_int(0)
+    k = lib().mxfp6_plan_kernel(out_type, M, N, Kp, (C.c_int * 4)(*tile), splits, a_layout,
+                                packed_bytes(Kp) if A_row_bytes is None else A_row_bytes,
+                                C.byref(w), C.byref(nt))
+    if k < 0:
+        raise ValueError(f"no such plan: {M}x{N}x{Kp} tile {tuple(tile)} splits {splits}")
+    return TILE_KERNELS[k], w.value, bool(nt.value)
 
 
 def plan_workspace_size(M, N, Kp, splits, a_repack):

@@ -1,0 +1,67 @@
+"""mxfp6_plan_kernel, from the rules that the launches act on (csrc/tile_dispatch.hpp): which kernel a plan's
+tile runs on, against the recorded times of the candidates."""
+import math
+import os
+
+import pytest
+
+PROFILE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "profiles",
+                       "skinny_tiles_on_row_major_a.txt")
+
+
+def _skinny_times():
+    with open(PROFILE) as f:
+        for line in f:
+            if not line.startswith("#"):
+                v = line.split()
+                yield [int(x) for x in v[:7]], dict(zip(("slab", "stream", "wide"), map(float, v[7:])))
+
+
+def _kernel(mx, M, N, K, MT, NT, S, **kw):
+    return mx.plan_kernel(mx.OUT_BF16, M, N, mx.kpad(K), (MT, NT, MT // 32, NT // 128), S, **kw)
+
+
+def test_skinny_tiles_run_on_the_faster_kernel(mx):
+    """Of the recorded plans none runs slower on the kernel it is given than on the slab kernel (which
+    the tiles ran on before, A repacked or not), nor more than 1.4 times the faster one of stream and
+    wide, 1% on average."""
+    over = []
+    for (M, N, K, MT, NT, S, rp), t in _skinny_times():
+        us = t[_kernel(mx, M, N, K, MT, NT, S)[0]]
+        assert us <= 1.03 * t["slab"], (M, N, K, MT, NT, S, t)
+        over.append(us / min(t["stream"], t["wide"]))
+        assert over[-1] < 1.4, (M, N, K, MT, NT, S, t)
+    assert len(over) > 400 and math.exp(sum(map(math.log, over)) / len(over)) < 1.01
+
+
+@pytest.mark.parametrize("MT,NT", [(32, 128), (32, 256), (64, 128), (64, 256)])
+def test_one_row_of_tiles_is_streamed(mx, MT, NT):
+    """A wide tile on one row of skinny tiles would be half to 31/32 repeated rows, however many
+    columns and segments there are."""
+    for N in (256, 4096, 28672, 32768, 65536, 102272):
+        for M in (1, MT // 2 + 1, MT):
+            for S in (1, 3, 8, 16):
+                assert _kernel(mx, M, N, 28672, MT, NT, S)[0] == "stream", (M, N, S)
+
+
+def test_long_rows_keep_the_tile(mx):
+    """128 row offsets of the wide tile stay within 31 bits: longer rows run on the 32- and 64-row tiles."""
+    args = (4096, 8192, 4096, 64, 256, 1)
+    assert _kernel(mx, *args)[0] == "wide"
+    assert _kernel(mx, *args, A_row_bytes=2**31 // 127 // 4 * 4)[0] == "wide"
+    assert _kernel(mx, *args, A_row_bytes=2**31 // 127 // 4 * 4 + 4)[0] == "stream"
+
+
+def test_other_layouts_and_tiles(mx):
+    k = lambda tile, layout, S=1: mx.plan_kernel(mx.OUT_F16, 256, 6144, 4224, tile, S, layout)[0]  # noqa: E731
+    assert k((64, 256, 2, 2), mx.A_REPACK) == k((32, 128, 1, 1), mx.A_PRESHUFFLED) == "slab"
+    assert k((128, 128, 2, 2), mx.A_ROWS) == k((256, 256, 4, 4), mx.A_ROWS) == "slab"
+    assert k((256, 192, 4, 3), mx.A_ROWS) == "slab"
+    assert k((128, 256, 4, 2), mx.A_ROWS) == k((128, 384, 4, 3), mx.A_ROWS) == "band"
+    assert k((128, 256, 4, 2), mx.A_REPACK) == "wide"
+    assert k((32, 32, 1, 1), mx.A_ROWS, 8) == "tiny"
+    for bad in ((256, 128, 4, 2), (64, 64, 2, 2)):
+        with pytest.raises(ValueError):
+            k(bad, mx.A_ROWS)
+    with pytest.raises(ValueError):
+        k((64, 256, 2, 2), mx.A_ROWS, 23)

@@ -14,6 +14,11 @@ SKINNY = [(32, 128, 1, 1), (32, 256, 1, 2), (64, 128, 2, 1), (64, 256, 2, 2)]
 T3 = {"dist_a": mx.DIST_STUDENT_T3, "dist_b": mx.DIST_STUDENT_T3}
 
 
+def runs_wide(dp, out_type, S):
+    p = dp.p
+    return mx.plan_kernel(out_type, p.M, p.N, p.Kp, dp.tile, S, A_row_bytes=p.a_row_bytes)[0] == "wide"
+
+
 def same(a, b):
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
@@ -23,19 +28,21 @@ def same(a, b):
 def test_bitwise_equals_direct(tile, K, S):
     """One to eight K-tiles (its short paths, which two B groups a wave end at two K-tiles, and its
     main loop), split and not, the last tile row partly past M."""
-    M, N = 2112 if S == 1 else 1088, 2048  # 136 or 144 workgroups of 128 x 256
+    M, N = 2112 if S == 1 else 1088, 2304  # 153 or 162 workgroups of 128 x 256
     p = checks.spread_scales(mx.make_problem(M, N, K // 32 * 32, **T3, seed=K), seed=K)
     dp = g.DevProblem(p, tile)
+    assert runs_wide(dp, mx.OUT_F32, S)
     same(g.run_explicit(dp, mx.OUT_F32, splits=S), g.run_direct(dp, mx.OUT_F32, splits=S))
 
 
 @pytest.mark.parametrize("tile", SKINNY)
-@pytest.mark.parametrize("M,N,K,S", [(2017, 2049, 800, 1), (1000, 4100, 192, 1), (97, 17000, 700, 2)])
+@pytest.mark.parametrize("M,N,K,S", [(2017, 2049, 800, 1), (1000, 4700, 192, 1), (97, 19000, 700, 2)])
 @pytest.mark.parametrize("out_type", [mx.OUT_F32, mx.OUT_F16])
 def test_ragged_equals_slab(tile, M, N, K, S, out_type):
     K = K // 32 * 32
     p = checks.spread_scales(mx.make_problem(M, N, K, **T3, seed=M + K), seed=M + K)
     dp = g.DevProblem(p, tile)
+    assert runs_wide(dp, out_type, S)
     same(g.run_explicit(dp, out_type, splits=S), g.run_explicit(dp, out_type, splits=S, a_layout=1))
 
 
@@ -45,4 +52,5 @@ def test_routed_repack_plans(M, N, K):
     tile, S, rp = mx.gemm_plan(mx.OUT_F32, M, N, p.Kp, mx.preferred_workspace_size(M, N, p.Kp))
     assert rp and tile[0] <= 64
     dp = g.DevProblem(p, tile)
+    assert runs_wide(dp, mx.OUT_F32, S)
     same(g.run_routed(dp, mx.OUT_F32), g.run_explicit(dp, mx.OUT_F32, splits=S, a_layout=1))
