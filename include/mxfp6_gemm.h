@@ -131,10 +131,8 @@ int mxfp6_gemm_explicit(int out_type, int M, int N, int Kp, const int tile[4], i
                         const uint8_t* dsB, void* dD, int A_row_bytes, void* ws, size_t ws_bytes,
                         void* stream);
 
-/* Whether the routed plan for (M, N, Kp) has room for a repacked A in its preferred workspace (gemm()
- * repacks A there, or, on 32- and 64-row tiles with many workgroups, reads the rows as they are
- * where that is faster: the same bits). No counterpart in the reference (its kernels read A
- * row-major). */
+/* Whether gemm() repacks A for (M, N, Kp) when its workspace allows (never on the 32- and 64-row tiles).
+ * No counterpart in the reference (its kernels read A row-major). */
 int mxfp6_gemm_repacks_a(int M, int N, int Kp);
 
 /* Measured plan selection. No counterpart in the reference (its router is a fixed rule).
@@ -167,7 +165,8 @@ void mxfp6_gemm_tune_reset(void);
  * file cannot be written. mxfp6_gemm_tune_load adds such a file's plans to the table, so that a
  * serving process can start with the plans an earlier run measured: a plan is taken only if its
  * tile is implemented, its split fits the shape and its scale grouping is the one choose_tile
- * returns for the shape on this device; *loaded and *skipped (may be NULL) count the lines taken
+ * returns for the shape on this device (a 32- or 64-row tile's on row-major A, whatever its line says of
+ * A); *loaded and *skipped (may be NULL) count the lines taken
  * and left. MXFP6_ERR_ARG when the file cannot be read. No counterpart in the reference. */
 int mxfp6_gemm_tune_save(const char* path, int* count);
 int mxfp6_gemm_tune_load(const char* path, int* loaded, int* skipped);

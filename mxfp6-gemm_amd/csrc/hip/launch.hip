@@ -164,12 +164,6 @@ extern "C" int mxfp6_hip_has_tile(int MT, int NT, int mpw, int npw) {
     return tile_supported(MT, NT, mpw, npw) ? 1 : 0;
 }
 
-extern "C" int mxfp6_hip_prefers_rows(int M, int N, int splits, int MT) {
-    const int reported = mxfp6_hip_device_cus();
-    const long cus = reported > 0 ? reported : 256;
-    return MT <= 64 && 5L * ((M + 127) / 128) * ((N + 255) / 256) * splits >= 2 * cus ? 1 : 0;
-}
-
 // Rows of the tiled scale layout: dim rounded up to whole groups of 32 * group rows.
 static int rows_in_groups(int dim, int group) {
     return (dim + 32 * group - 1) / (32 * group) * (32 * group);

@@ -66,10 +66,6 @@ void* mxfp6_hip_scratch(size_t* bytes);
 /* Clock sample (see mxfp6_clock_sample_async in include/mxfp6_gemm.h). 0 ok, 2 launch error. */
 int mxfp6_hip_clock_sample(uint64_t* out, int nwg, void* stream);
 
-/* 1 when a plan on this tile that repacks A first runs faster on row-major A (the skinny tiles on
- * enough workgroups), else 0. The output bits are the same. */
-int mxfp6_hip_prefers_rows(int M, int N, int splits, int MT);
-
 /* Compute units of the current HIP device (hipDeviceAttributeMultiprocessorCount, read once per
  * device), or 0 when the runtime reports no device. */
 int mxfp6_hip_device_cus(void);

@@ -101,6 +101,9 @@ bool is_wide(const TileChoice& tc) {
            (tc.MT == 256 && tc.NT == 256 && tc.MPW == 4 && tc.NPW == 2);
 }
 
+// The 32- and 64-row tiles; gemm() runs them on row-major A.
+bool is_skinny(const TileChoice& tc) { return tc.MT <= 64; }
+
 double plan_time_us(const TileChoice& tc, int M, int N, int Kp, int S, bool repack, int CUS) {
     const long wg = (long)((M + tc.MT - 1) / tc.MT) * ((N + tc.NT - 1) / tc.NT) * S;
     const int occ = (tc.NT == 128 && (tc.MT == 128 || tc.MT == 32)) ? 2 : 1;  // per CU (LDS)
@@ -235,6 +238,11 @@ Plan best_plan(int M, int N, int Kp, int cus) {
             best_t = t;
         }
     });
+    // The model knows the skinny tiles as the slab kernel ran them, on A repacked where that was faster.
+    // Row-major A runs on other kernels now (tile_dispatch.hpp): as fast or up to 2.8 times faster on 241
+    // of 242 measured plans that would have repacked (profiles/skinny_tiles_on_row_major_a.txt;
+    // 320 x 23808 x 12672 144.4 us repacked, 146.6 on the rows), with no workspace for A.
+    if (is_skinny(best.tc)) best.repack = false;
     return best;
 }
 
@@ -468,12 +476,9 @@ int kernel_for(const TileChoice& tc) {
 
 Plan plan_for(int out_type, int M, int N, int Kp, size_t ws_bytes, bool* unsplit);
 
-// The A layout a plan is launched with: a plan that repacks A reads the rows as they are where the
-// launch layer has a faster kernel for them (the plan's workspace is then not touched for A).
-int layout_of(const Plan& pl, int M, int N, int kernel) {
-    return pl.repack && kernel == MXFP6_KERNEL_TILE && !mxfp6_hip_prefers_rows(M, N, pl.S, pl.tc.MT)
-               ? MXFP6_A_REPACK
-               : MXFP6_A_ROWS;
+// The A layout a plan is launched with.
+int layout_of(const Plan& pl, int kernel) {
+    return pl.repack && kernel == MXFP6_KERNEL_TILE ? MXFP6_A_REPACK : MXFP6_A_ROWS;
 }
 
 int gemm_checked(int out_type, int M, int N, int Kp, const void* dA, const void* dBsh,
@@ -491,8 +496,8 @@ int gemm_checked(int out_type, int M, int N, int Kp, const void* dA, const void*
                      M, N, Kp, splitk_segments(M, N, Kp), workspace_bytes(M, N, Kp), ws_bytes);
     const int kernel = kernel_for(pl.tc);
     if (kernel != MXFP6_KERNEL_TILE && (M % 64 != 0 || N % 64 != 0)) return MXFP6_ERR_TILE;
-    return run(out_type, M, N, Kp, pl.tc, pl.S, layout_of(pl, M, N, kernel), kernel, dA, dBsh, dsA,
-               dsB, dD, A_row_bytes, ws, stream);
+    return run(out_type, M, N, Kp, pl.tc, pl.S, layout_of(pl, kernel), kernel, dA, dBsh, dsA, dsB,
+               dD, A_row_bytes, ws, stream);
 }
 
 // The plan gemm() runs for a workspace of ws_bytes: a measured plan of the shape when the
@@ -528,7 +533,7 @@ int tune_launch(void* ctx) {
     const TuneCall& c = *static_cast<const TuneCall*>(ctx);
     const int kernel = kernel_for(c.plan.tc);
     return run(c.out_type, c.M, c.N, c.Kp, c.plan.tc, c.plan.S,
-               layout_of(c.plan, c.M, c.N, kernel), kernel, c.dA, c.dBsh, c.dsA, c.dsB, c.dD,
+               layout_of(c.plan, kernel), kernel, c.dA, c.dBsh, c.dsA, c.dsB, c.dD,
                c.A_row_bytes, c.ws, c.stream);
 }
 }  // namespace
@@ -568,6 +573,7 @@ int tune(int out_type, int M, int N, int Kp, const void* dA, const void* dBsh, c
         if (tc.MT == routed.tc.MT && tc.NT == routed.tc.NT && S == routed.S && rp == routed.repack)
             return;
         if (tc.MPW != routed.tc.MPW || tc.NPW != routed.tc.NPW) return;
+        if (rp && is_skinny(tc)) return;  // as best_plan
         if (kernel_for(tc) != MXFP6_KERNEL_TILE) return;
         if (!plan_fits(M, N, Kp, S, rp, ws_bytes)) return;
         ranked.push_back({plan_time_us(tc, M, N, Kp, S, rp, cus), {tc, S, rp}});
@@ -658,7 +664,7 @@ int tune_save(const char* path, int* count) {
 // Adds the plans of a tune_save file to the table. A line is taken only if it names a tile the
 // kernels implement, a split the shape allows, and the scale grouping choose_tile returns for the
 // shape on this device (the caller's scales are tiled for that grouping); others are counted as
-// skipped, as are malformed lines.
+// skipped, as are malformed lines. A plan of a 32- or 64-row tile is taken on row-major A (best_plan).
 int tune_load(const char* path, int* loaded, int* skipped) {
     FILE* f = std::fopen(path, "r");
     if (f == nullptr) return MXFP6_ERR_ARG;
@@ -684,7 +690,7 @@ int tune_load(const char* path, int* loaded, int* skipped) {
             n_skip++;
             continue;
         }
-        store_tuned(ot, M, N, Kp, {tc, S, rp != 0});
+        store_tuned(ot, M, N, Kp, {tc, S, rp != 0 && !is_skinny(tc)});
         n_ok++;
     }
     std::fclose(f);

@@ -142,13 +142,14 @@ def tiny_segments(M, N, Kp):
 
 def best_plan(c, M, N, Kp):
     """(tile, S, repack) with the least predicted time, as plan.cpp best_plan (the 32 x 32 tile's
-    rule first)."""
+    rule first; the 32- and 64-row tiles read row-major A, whatever the model says)."""
     if tiny_routed(M, N, Kp):
         return (TINY, tiny_segments(M, N, Kp), False)
     cands = candidates(M, N, Kp)
     if not cands:
         return ((128, 128, 2, 2), 1, False)
-    return cands[_pick([plan_time_us(c, t, M, N, Kp, S, rp) for t, S, rp in cands])]
+    t, S, rp = cands[_pick([plan_time_us(c, t, M, N, Kp, S, rp) for t, S, rp in cands])]
+    return (t, S, rp and t[0] > 64)
 
 
 def load(paths):

@@ -65,3 +65,36 @@ def test_other_layouts_and_tiles(mx):
             k(bad, mx.A_ROWS)
     with pytest.raises(ValueError):
         k((64, 256, 2, 2), mx.A_ROWS, 23)
+
+
+def test_plans_say_what_runs(mx):
+    """The recorded plans that repacked A for the slab kernel read its rows now: every query says so, the
+    workspace holds the K segments only, and with those bytes the plan is the same one."""
+    n = 0
+    for (M, N, K, MT, NT, S, rp), _ in _skinny_times():
+        if not rp:
+            continue
+        Kp, tile = mx.kpad(K), (MT, NT, MT // 32, NT // 128)
+        assert not mx.repacks_a(M, N, Kp), (M, N, K)
+        split = 4 * S * M * N if S > 1 else 0
+        assert mx.workspace_size(M, N, Kp) == split
+        assert mx.preferred_workspace_size(M, N, Kp) == -(-split // 256) * 256
+        for ws in (split, 1 << 40):
+            assert mx.gemm_plan(mx.OUT_F16, M, N, Kp, ws) == (tile, S, False), (M, N, K, ws)
+        n += 1
+    assert n > 200
+
+
+def test_loaded_skinny_plan_reads_rows(mx, tmp_path):
+    M, N, Kp = 3616, 5120, mx.kpad(4096)
+    tile = mx.choose_tile(M, N, Kp)
+    assert tile[0] <= 64
+    f = tmp_path / "plans.txt"
+    f.write_text(" ".join(map(str, (1, M, N, Kp, *tile, 1, 1))) + "\n")
+    mx.tune_reset()
+    try:
+        assert mx.tune_load(str(f)) == (1, 0)
+        assert mx.tuned_plan(1, M, N, Kp) == (tuple(tile), 1, False)
+        assert mx.gemm_plan(1, M, N, Kp, 0) == (tuple(tile), 1, False)
+    finally:
+        mx.tune_reset()
