@@ -169,14 +169,29 @@ static int rows_in_groups(int dim, int group) {
     return (dim + 32 * group - 1) / (32 * group) * (32 * group);
 }
 
+static int prep_chunks(int cols) {
+    return ((cols + 31) / 32 + PREP_BLKS_PER_WAVE - 1) / PREP_BLKS_PER_WAVE;
+}
+
+// Fewer waves a CU once there are more than 32 for each (1024 x 16128, 32 a CU: 14.6 us against 14.4;
+// 512 x 16128: 9.2 against 8.7; above, prep_kernel.hpp) and each has more than 1024 values on average: a
+// wave of a short row keeps few loads in flight, and 12 of them leave the memory idle
+// (profiles/prep_rows_waves_in_flight.txt: 39040 x 256 32.1 us against 21.4 with as many as fit, 65408 x
+// 512 55.8 and 35.9, 9760 x 1024 13.1 and 12.0; 26144 x 1280 32.0 and 34.4, 16096 x 2080 44.2 and 45.4).
+extern "C" int mxfp6_hip_prep_few_waves(int rows, int cols) {
+    const int reported = mxfp6_hip_device_cus(), chunks = prep_chunks(cols);
+    return (size_t)rows * chunks > 32 * (size_t)(reported > 0 ? reported : 256) && cols > 1024L * chunks
+               ? 1
+               : 0;
+}
+
 extern "C" int mxfp6_hip_quantize_rows(const float* x, int rows, int cols, int nblk, void* packed,
                                        size_t row_bytes, int preshuffled, uint8_t* scales,
                                        int scale_mode, int ncols, int group, int Kp, void* stream) {
     // one wave per (row, 64 value blocks); the last chunk of a row also writes its K-tail blocks;
     // one block per lane: more, smaller one-wave workgroups beat 2 or 4 blocks per lane (8192^2:
     // 76 us against 100 and 163 us; the LDS per workgroup bounds the waves per CU)
-    const int vblk = (cols + 31) / 32;
-    const int chunks = (vblk + PREP_BLKS_PER_WAVE - 1) / PREP_BLKS_PER_WAVE;
+    const int chunks = prep_chunks(cols);
     const int rows32 = (rows + 31) / 32 * 32;
     int rows_out = scale_mode ? rows_in_groups(rows, group) : rows;
     if (preshuffled) rows_out = std::max(rows_out, rows32);
@@ -194,10 +209,7 @@ extern "C" int mxfp6_hip_quantize_rows(const float* x, int rows, int cols, int n
                                        rows32, so));
     }
     const dim3 grid((unsigned)((size_t)rows_out * chunks));
-    // fewer waves a CU once there are more than 32 for each (1024 x 16128, 32 a CU: 14.6 us against
-    // 14.4; 512 x 16128: 9.2 against 8.7; above, prep_kernel.hpp)
-    const int reported = mxfp6_hip_device_cus();
-    const bool few = (size_t)rows_out * chunks > 32 * (size_t)(reported > 0 ? reported : 256);
+    const bool few = mxfp6_hip_prep_few_waves(rows_out, cols) != 0;
     return status_of(launch_kernel(few ? prep_rows_kernel<true> : prep_rows_kernel<false>, grid,
                                    dim3(64), st, x, cols, nblk, po, so, chunks, rows));
 }

@@ -78,6 +78,10 @@ int mxfp6_hip_time(int (*launch)(void* ctx), void* ctx, void* stream, int warm, 
 /* Whether the tile kernel has an instantiation for MT x NT with scale grouping (mpw, npw). */
 int mxfp6_hip_has_tile(int MT, int NT, int mpw, int npw);
 
+/* 1 where mxfp6_hip_quantize_rows keeps fewer waves a CU in flight than fit, for `rows` rows written
+ * (whole scale groups where tiled) of cols values. */
+int mxfp6_hip_prep_few_waves(int rows, int cols);
+
 /* Quantisation and layout kernels (csrc/hip/prep_kernel.hpp). All return 0 ok, 2 launch error.
  *
  * Row-major float x[rows][cols] (4-byte aligned; 16-byte aligned with cols % 4 == 0 reads float4):

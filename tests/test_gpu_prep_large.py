@@ -19,10 +19,13 @@ def out(n):
     return torch.full((n,), 0x5A, dtype=torch.uint8, device="cuda")
 
 
-@pytest.mark.parametrize("rows,cols,shift", [(8256, 2048, 0), (8224, 2049, 0), (4160, 4100, 1),
-                                             (8256, 31, 3), (2080, 16127, 0)])
-def test_rows(rows, cols, shift):
-    """More than 32 waves a CU (FEW), rows of any length and inputs of any 4-byte alignment."""
+@pytest.mark.parametrize("rows,cols,shift,few", [(8256, 2048, 0, 1), (8224, 2049, 0, 1), (4160, 4100, 1, 1),
+                                                 (8256, 1025, 2, 1), (8256, 1024, 2, 0), (8256, 31, 3, 0),
+                                                 (2080, 16127, 0, 1)])
+def test_rows(rows, cols, shift, few):
+    """More than 32 waves a CU, in fewer at a time (FEW) where a wave has more than 1024 values, rows of any
+    length and inputs of any 4-byte alignment."""
+    assert mx.lib().mxfp6_hip_prep_few_waves(rows, cols) == few
     x = torch.empty(rows * cols + 4, device="cuda")[shift:shift + rows * cols].view(rows, cols)
     x.copy_(values(rows, cols, cols))
     Kp = mx.kpad(cols)
