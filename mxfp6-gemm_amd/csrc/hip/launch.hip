@@ -218,12 +218,10 @@ extern "C" int mxfp6_hip_prepare_b(const float* B, int K, int N, int Kp, int gro
                                    uint8_t* tiled, void* stream) {
     const int NG = rows_in_groups(N, group);
     const unsigned nchunks = (unsigned)((NG + PREP_THREADS - 1) / PREP_THREADS), kchunks = (unsigned)(Kp / 32);
-    // B and its codes against half of the 256 MiB last-level cache
-    const double half = 128.0 * (1 << 20), values = (double)K * N;
-    auto k = 4 * values < half     ? prep_b_kernel<false, false>
-             : 0.75 * values < half ? prep_b_kernel<true, false>
-                                    : prep_b_kernel<true, true>;
-    return status_of(launch_kernel(k, dim3(nchunks * kchunks), dim3(PREP_THREADS),
+    // B against half of the 256 MiB last-level cache
+    const bool few = 4.0 * K * N >= 128.0 * (1 << 20);
+    return status_of(launch_kernel(few ? prep_b_kernel<true> : prep_b_kernel<false>,
+                                   dim3(nchunks * kchunks), dim3(PREP_THREADS),
                                    static_cast<hipStream_t>(stream), B, K, N, NG, Kp, group,
                                    static_cast<uint8_t*>(bsh), tiled, (int)nchunks));
 }

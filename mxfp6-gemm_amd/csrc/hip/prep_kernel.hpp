@@ -357,9 +357,10 @@ __global__ void __launch_bounds__(64 * PSH_SLABS)
 // nontemporal loads: with fewer rows' pieces in flight the memory serves them faster, and B is not
 // read again (8192 x 4096 34.0 -> 28.0 us, 8192 x 8192 62.0 -> 52.3, 8192 x 14336 107.5 -> 95.9;
 // FEW alone 31.4, 58.1 and 103.9; B that the last-level cache may hold loses by nontemporal loads,
-// 8192 x 2048 12.8 -> 15.2). NTS stores the codes nontemporally too, where they would fill half that
-// cache: 8192 x 28672 218.9 -> 205.0 with FEW, 198.5 with both.
-template <bool FEW, bool NTS>
+// 8192 x 2048 12.8 -> 15.2). The codes are stored the ordinary way: past the caches 8192 x 28672 took 197
+// us in place of 206 by itself, but the GEMM that reads them next lost more (with it, M = 32 240 -> 246,
+// M = 256 259 -> 264, M = 2048 477 -> 514; 8192 x 22016: 186 -> 203, 209 -> 222, 373 -> 405).
+template <bool FEW>
 __global__ void __launch_bounds__(PREP_THREADS)
     prep_b_kernel(const float* __restrict__ B, int K, int N, int NG, int Kp, int group,
                   uint8_t* __restrict__ bsh, uint8_t* __restrict__ tiled, int nchunks) {
@@ -386,15 +387,8 @@ __global__ void __launch_bounds__(PREP_THREADS)
     if (n < (N + 31) / 32 * 32) {
         const int k64n = Kp / 64, t = (n & 31) + ((c & 1) << 5);
         uint8_t* tile = bsh + ((size_t)(n >> 5) * k64n + (c >> 1)) * OPBLK_BYTES;
-        const v4i lo = {(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-        const v2i hi = {(int)w[4], (int)w[5]};
-        if constexpr (NTS) {
-            __builtin_nontemporal_store(lo, reinterpret_cast<v4i*>(tile + 16 * t));
-            __builtin_nontemporal_store(hi, reinterpret_cast<v2i*>(tile + 1024 + 8 * t));
-        } else {
-            *reinterpret_cast<v4i*>(tile + 16 * t) = lo;
-            *reinterpret_cast<v2i*>(tile + 1024 + 8 * t) = hi;
-        }
+        *reinterpret_cast<v4i*>(tile + 16 * t) = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+        *reinterpret_cast<v2i*>(tile + 1024 + 8 * t) = v2i{(int)w[4], (int)w[5]};
     }
     put_tiled_scale(tiled, n, c, group, Kp / 192, code);
 }

@@ -1,4 +1,4 @@
-"""The preparation kernels past the sizes where they bound the waves in flight and load (and store)
+"""The preparation kernels past the sizes where they bound the waves in flight and load B
 nontemporally: the bytes of the whole operand against those of its pieces, each under those sizes
 (rows of A are independent, and so are the 32-column blocks of B's layout)."""
 import pytest
