@@ -214,13 +214,20 @@ extern "C" int mxfp6_hip_quantize_rows(const float* x, int rows, int cols, int n
                                    dim3(64), st, x, cols, nblk, po, so, chunks, rows));
 }
 
+// B against half of the 256 MiB last-level cache, and columns that fill more than 3/5 of their 256-column
+// workgroups: with fewer the workgroups in flight load too little (profiles/prep_b_waves_in_flight.txt: N =
+// 40, 160 MB, 40.3 -> 73.5 us with FEW, N = 300, 240 MB, 69.9 -> 71.4; N = 317, 134 MB, 38.7 -> 39.3, N = 384,
+// 162 MB, 42.1 -> 36.6).
+extern "C" int mxfp6_hip_prep_b_few(int K, int N) {
+    const long columns = (N + (long)PREP_THREADS - 1) / PREP_THREADS * PREP_THREADS;
+    return 4.0 * K * N >= 128.0 * (1 << 20) && 5L * N > 3 * columns ? 1 : 0;
+}
+
 extern "C" int mxfp6_hip_prepare_b(const float* B, int K, int N, int Kp, int group, void* bsh,
                                    uint8_t* tiled, void* stream) {
     const int NG = rows_in_groups(N, group);
     const unsigned nchunks = (unsigned)((NG + PREP_THREADS - 1) / PREP_THREADS), kchunks = (unsigned)(Kp / 32);
-    // B against half of the 256 MiB last-level cache
-    const bool few = 4.0 * K * N >= 128.0 * (1 << 20);
-    return status_of(launch_kernel(few ? prep_b_kernel<true> : prep_b_kernel<false>,
+    return status_of(launch_kernel(mxfp6_hip_prep_b_few(K, N) ? prep_b_kernel<true> : prep_b_kernel<false>,
                                    dim3(nchunks * kchunks), dim3(PREP_THREADS),
                                    static_cast<hipStream_t>(stream), B, K, N, NG, Kp, group,
                                    static_cast<uint8_t*>(bsh), tiled, (int)nchunks));

@@ -95,6 +95,9 @@ int mxfp6_hip_quantize_rows(const float* x, int rows, int cols, int nblk, void* 
                             size_t row_bytes, int preshuffled, uint8_t* scales, int scale_mode,
                             int ncols, int group, int Kp, void* stream);
 
+/* 1 where mxfp6_hip_prepare_b keeps four workgroups a CU in flight and loads B nontemporally. */
+int mxfp6_hip_prep_b_few(int K, int N);
+
 /* Row-major float B[K][N] -> preshuffled B^T at Kp (N/32 * Kp/64 * 1536 bytes) and its scales
  * in the tile_scale(group, 3) layout at Kp. N % (32 * group) == 0. */
 int mxfp6_hip_prepare_b(const float* B, int K, int N, int Kp, int group, void* bsh,

@@ -44,10 +44,11 @@ def test_rows(rows, cols, shift, few):
         assert torch.equal(p[r0:r0 + 1031], pp) and torch.equal(s[r0:r0 + 1031], ps)
 
 
-@pytest.mark.parametrize("K,N", [(8192, 4096), (4099, 8256), (16384, 12288)])
+@pytest.mark.parametrize("K,N", [(8192, 4096), (4099, 8256), (16384, 12288), (110000, 330)])
 @pytest.mark.parametrize("group", [2, 3])
 def test_b(K, N, group):
-    """B of half the last-level cache and more, and (16384 x 12288) codes of that."""
+    """B of half the last-level cache and more."""
+    assert mx.lib().mxfp6_hip_prep_b_few(K, N)
     B = values(K, N, N)
 
     def prepare(b):
