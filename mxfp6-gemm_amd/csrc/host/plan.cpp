@@ -421,7 +421,7 @@ bool streams_output(int out_type, int M, int N, int Kp, const TileChoice& tc, in
     const double out = (double)M * N * (out_type == 0 ? 4 : 2);  // FP32 or a 16-bit type
     if (in > LLC_BYTES) return false;
     return in + out > STREAM_FOOTPRINT_BYTES ||
-           (in + out > LLC_BYTES / 2 &&
+           (out_type != 0 && in + out > LLC_BYTES / 2 &&
             out >= (in + out <= STREAM_MID_BYTES ? STREAM_MID_RATIO : STREAM_D_RATIO) * in);
 }
 

@@ -31,20 +31,23 @@ constexpr double PLAN_MIN_GAIN = 0.01;     // lead a more complex plan needs ove
 // repacked A: "in", at most MI355X's 256 MiB last-level cache) and writes ("out"):
 //   in + out > STREAM_FOOTPRINT_BYTES: D no longer evicts the operands the tiles re-read (6-22% faster,
 //   8192x16384x2048, 4096x51200x1024, 16384x16384x4096, 1024x102272x2048, 2048x102272x1024; no
-//   difference once the operands alone exceed the cache, 2048x102272x4096);
-//   in + out from half the cache to STREAM_MID_BYTES, D no less than STREAM_MID_RATIO of in: two such
-//   calls in a row, on operands and outputs of their own as a program's layers are, no longer fit the
-//   cache together, and the plain stores of one wait for the other's D to be written back. Plain ->
-//   streamed with the epilogue's full-line stores, three sets in turn (the same set over and over):
-//   8192x8192x2048 120.5 -> 103.6 us (109.4 -> 103.5), 8192x8192x4096 198.8 -> 166.9 (167.7 -> 167.4),
-//   4096x14336x4096 188.4 -> 154.5 (156.4 -> 154.1), 8192x5120x8192 243.7 -> 202.1 (203.2 -> 201.4),
-//   1024x28672x4096 98.8 -> 97.2 (78.8 -> 77.3), FP32 4096x6144x4096 90.4 -> 75.6 (73.8 -> 74.8) and
-//   4096x8192x2048 74.0 -> 70.9 (68.1 -> 71.0); 16-bit outputs: 16 of 16 shapes not slower either
-//   way. The gain ends at 240 MB (8192^3 340.8 -> 326.7, 300.3 -> 298.3), below half the cache
-//   it is -2 to 4% (4096x8192x2048 53.2 -> 54.5, 8192x6144x1024 60.5 -> 58.1). The ratio keeps
-//   out the plans that run as 128-row bands (stream_kernel.hpp), whose D is small;
-//   past that up to STREAM_FOOTPRINT_BYTES, D at least STREAM_D_RATIO times in (short K):
-//   16384x8192x512 155.8 -> 117.5 us (130.6 -> 116.1).
+//   difference once the operands alone exceed the cache, 2048x102272x4096), and a kernel that reads D next
+//   would not find it cached either (the pair 5-10% faster on 8192x16384x2048 and 4096x28672x4096);
+//   16-bit D, in + out from half the cache to STREAM_MID_BYTES, D no less than STREAM_MID_RATIO of in: two
+//   such calls in a row no longer fit the cache together, and the plain stores of one wait for the other's
+//   D to be written back. profiles/gemm_d_stores_with_a_reader.txt, 17 to 25 shapes, streamed against plain:
+//   the GEMM alone takes 0.88 times as long where operands and D rotate (8192x8192x1024 86.6 -> 70.2 us,
+//   8192x8192x4096 202.9 -> 175.4), 0.94 where D is one buffer (0.83-1.04), and with a kernel after it that
+//   reads D and writes as much 0.965 and 0.98 (0.92-1.04). A kernel that only reads D gives the gain back:
+//   0.985 where D rotates, 1.065 where it is one buffer (8192x8192x1024 97.2 -> 113.2). The ratio
+//   keeps out the plans that run as 128-row bands (tile_dispatch.hpp), whose D is small. STREAM_MID_BYTES is
+//   not where the gain ends: from there to STREAM_FOOTPRINT_BYTES streaming measured 0.87 alone and 0.95 with
+//   a kernel that reads and writes (8192^3 346.2 -> 329.6 and 388.3 -> 380.2; only reading, 370.7 -> 378.3);
+//   plain stores have stayed there but for D of at least STREAM_D_RATIO times in (short K: 8192x14336x512
+//   96.5 -> 84.9).
+// FP32 D up to STREAM_FOOTPRINT_BYTES is stored the ordinary way: what reads it next is prepare_a, and the pair
+// is 3-8% slower with D streamed (4096x8192x2048 96.7 -> 105.5 us, one D 85.6 -> 100.1), as the GEMM alone
+// is where D is one buffer (60.2 -> 71.1).
 constexpr double LLC_BYTES = 268435456.0;
 constexpr double STREAM_FOOTPRINT_BYTES = 280e6;
 constexpr double STREAM_MID_BYTES = 236e6;

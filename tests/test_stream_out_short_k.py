@@ -1,6 +1,6 @@
-"""Unsplit plans on wide tiles whose operands and D fill half the 256 MiB last-level cache or more write
-D with nontemporal stores where D is at least 0.4 times the operands (up to 236 MB in all) or 8 times
-(above): the rule's edges, and the values against the direct kernel bit for bit."""
+"""Unsplit plans on wide tiles whose operands and 16-bit D fill half the 256 MiB last-level cache or more
+write D with nontemporal stores where D is at least 0.4 times the operands (up to 236 MB in all) or 8 times
+(above), FP32 D only past 280 MB: the rule's edges, and the values against the direct kernel bit for bit."""
 import pytest
 
 import checks
@@ -16,7 +16,10 @@ import mxfp6_amd as mx
     (256, 18432, 12288, mx.OUT_F32, False),   # D a tenth of the operands
     (8192, 12288, 3072, mx.OUT_BF16, False),  # 251 MB in all, D 4x
     (8192, 15360, 512, mx.OUT_BF16, True),    # 262 MB, D over 8x
-    (4096, 10240, 1024, mx.OUT_F32, True),    # 16-bit D would not fill half the cache
+    (4096, 10240, 1024, mx.OUT_F32, False),   # FP32 D of 168 MB: prepare_a finds it cached
+    (4096, 8192, 2048, mx.OUT_F32, False),
+    (4096, 16384, 512, mx.OUT_F32, False),    # 268 + 8 MB
+    (4096, 17408, 512, mx.OUT_F32, True),     # 285 + 8 MB
     (4096, 10240, 1024, mx.OUT_F16, False),
     (2048, 28672, 1024, mx.OUT_F16, True)])
 def test_rule(M, N, K, out_type, want):
@@ -27,7 +30,8 @@ def test_rule(M, N, K, out_type, want):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,out_type", [(8192, 8192, 1024, mx.OUT_BF16), (2048, 28672, 1344, mx.OUT_F16),
-                                            (4096, 10240, 960, mx.OUT_F32)])
+                                            (8192, 10240, 960, mx.OUT_F16),
+                                            (4096, 17408, 512, mx.OUT_F32)])
 def test_equals_direct_kernel(M, N, K, out_type):
     from gpu_util import DevProblem, run_direct, run_routed
     p = checks.spread_scales(mx.make_problem(M, N, K, seed=M + N + K), seed=K)
