@@ -352,8 +352,9 @@ def test_plan_cache_is_per_thread_and_transparent(mx):
 
 
 def test_streaming_rule(mx):
-    """D is written with nontemporal stores only by unsplit plans whose operands fit in the
-    256 MiB last-level cache while the operands and D together do not."""
+    """D is written with nontemporal stores only by unsplit plans whose operands fit in the 256 MiB
+    last-level cache; the cases here by whether the operands and D together do
+    (tests/test_stream_out_short_k.py has the 16-bit D that is streamed although they do)."""
     cases = [((8192, 8192, 8192), 1, False),     # everything fits
              ((2048, 1024, 105728), 1, False),   # split K: the reduce writes D
              ((2048, 51200, 1024), 1, False),    # 253 MB in all: fits

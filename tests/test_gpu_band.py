@@ -3,6 +3,7 @@
 bit the direct kernel's output, and on ragged shapes the wide kernel's on the repacked A."""
 import numpy as np
 import pytest
+import torch
 
 import checks
 import mxfp6_amd as mx
@@ -19,12 +20,13 @@ def same(a, b):
 
 
 @pytest.mark.parametrize("tile", WIDE)
-@pytest.mark.parametrize("M,N,K,S", [(128, 384, 1536, 1),    # two waves, a whole number of chunks
-                                     (256, 768, 1728, 1),    # nine K-tiles: a partial chunk
-                                     (512, 6144, 1536, 1),   # three waves
-                                     (512, 7680, 1600, 1),   # four, the last K-tile half values
-                                     (256, 1536, 4992, 3)])  # segments of nine and eight K-tiles
-def test_band_bitwise_equals_direct(tile, M, N, K, S):
+@pytest.mark.parametrize("M,N,K,S,waves", [(128, 384, 1536, 1, 2),    # a whole number of chunks
+                                           (256, 768, 1728, 1, 2),    # nine K-tiles: a partial chunk
+                                           (512, 6144, 1536, 1, 3),
+                                           (512, 7680, 1600, 1, 4),   # the last K-tile half values
+                                           (256, 1536, 4992, 3, 2)])  # segments of nine and eight K-tiles
+def test_band_bitwise_equals_direct(tile, M, N, K, S, waves):
+    assert mx.plan_kernel(mx.OUT_F32, M, N, mx.kpad(K), tile, S) == ("band", waves, False)
     seed = M + N + K
     p = checks.spread_scales(mx.make_problem(M, N, K, **T3, seed=seed), seed=seed)
     dp = g.DevProblem(p, tile)
@@ -39,14 +41,18 @@ def test_band_ragged_equals_wide(tile, M, N, K, S, out_type):
     K = K // 32 * 32
     p = checks.spread_scales(mx.make_problem(M, N, K, **T3, seed=M + K), seed=M + K)
     dp = g.DevProblem(p, tile)
+    assert mx.plan_kernel(out_type, M, N, p.Kp, tile, S, A_row_bytes=p.a_row_bytes)[0] == "band"
     same(g.run_explicit(dp, out_type, splits=S), g.run_explicit(dp, out_type, splits=S, a_layout=1))
 
 
-@pytest.mark.parametrize("M,N,Kp", [(250, 18432, 4992),    # B of a quarter of the last-level cache: five waves
-                                    (128, 24576, 7488)])   # half of it, one tile row: nontemporal loads
-def test_band_large_b_equals_wide(M, N, Kp):
-    import torch
+@pytest.mark.parametrize("M,N,Kp,waves,nt", [
+    (250, 18432, 4992, 5, False),   # B of a quarter of the last-level cache: five waves
+    (128, 24576, 7488, 3, True),    # half of it, one tile row: nontemporal loads
+    (123, 40950, 4416, 5, True)])   # both, masked
+@pytest.mark.parametrize("out_type,dtype", [(mx.OUT_F32, torch.float32), (mx.OUT_F16, torch.float16)])
+def test_band_large_b_equals_wide(M, N, Kp, waves, nt, out_type, dtype):
     tile = (128, 256, 4, 2)
+    assert mx.plan_kernel(out_type, M, N, Kp, tile) == ("band", waves, nt)
     gen = torch.Generator(device="cuda").manual_seed(5)
     b = lambda n, lo, hi: torch.randint(lo, hi, (n,), generator=gen, device="cuda", dtype=torch.uint8)  # noqa: E731
     row = mx.packed_bytes(Kp)
@@ -56,10 +62,10 @@ def test_band_large_b_equals_wide(M, N, Kp):
     for layout in (0, 1):
         n = max(4, mx.plan_workspace_size(M, N, Kp, 1, layout == 1))
         ws = torch.empty(n, dtype=torch.uint8, device="cuda")
-        d = torch.empty(M, N, device="cuda")
-        rc = mx.gemm_explicit(mx.OUT_F32, M, N, Kp, tile, 1, a.data_ptr(), bsh.data_ptr(), sa.data_ptr(),
+        d = torch.empty(M, N, dtype=dtype, device="cuda")
+        rc = mx.gemm_explicit(out_type, M, N, Kp, tile, 1, a.data_ptr(), bsh.data_ptr(), sa.data_ptr(),
                               sb.data_ptr(), d.data_ptr(), row, ws.data_ptr(), n, a_layout=layout)
         assert rc == 0, mx.STATUS.get(rc, rc)
         torch.cuda.synchronize()
-        D.append(d.cpu().numpy())
+        D.append(d.float().cpu().numpy())
     same(D[0], D[1])

@@ -46,11 +46,12 @@ def test_ragged_equals_slab(tile, M, N, K, S, out_type):
     same(g.run_explicit(dp, out_type, splits=S), g.run_explicit(dp, out_type, splits=S, a_layout=1))
 
 
-@pytest.mark.parametrize("M,N,K", [(3616, 5120, 4096), (1184, 25856, 1536), (576, 8192, 6016)])
-def test_routed_plans(M, N, K):
+@pytest.mark.parametrize("M,N,K,kernel", [(3616, 5120, 4096, "wide"), (1184, 25856, 1536, "wide"),
+                                          (576, 8192, 6016, "wide"), (1056, 1920, 17408, "stream")])
+def test_routed_plans(M, N, K, kernel):
     p = checks.spread_scales(mx.make_problem(M, N, K, **T3, seed=M), seed=M)
     tile, S, rp = mx.gemm_plan(mx.OUT_F32, M, N, p.Kp, mx.preferred_workspace_size(M, N, p.Kp))
     assert not rp and tile[0] <= 64
     dp = g.DevProblem(p, tile)
-    assert runs_wide(dp, mx.OUT_F32, S)
+    assert mx.plan_kernel(mx.OUT_F32, M, N, p.Kp, tile, S, A_row_bytes=p.a_row_bytes)[0] == kernel
     same(g.run_routed(dp, mx.OUT_F32), g.run_explicit(dp, mx.OUT_F32, splits=S, a_layout=1))
