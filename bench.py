@@ -92,9 +92,9 @@ CONFIGS = {
            (mx.DIST_STUDENT_T3, 1.0), "A,B ~ Student-t(3)"),
 }
 PROFILES = os.path.join(ROOT, "profiles")
-# the tiles run by wide_kernel (four waves side by side, B loaded into registers); the others by
-# slab_kernel
-WIDE_TILES = {(128, 512, 4, 4), (128, 384, 4, 3), (128, 256, 4, 2), (256, 256, 4, 2)}
+# the kernel that each answer of mx.plan_kernel runs
+KERNEL_NAMES = {"tiny": "tiny_kernel", "slab": "slab_kernel", "wide": "wide_kernel",
+                "stream": "stream_kernel", "band": "stream_kernel"}
 METRIC = "MXFP6 GEMM TFLOPs (FP16 out) and % of MXFP6 MFMA peak, 1xMI355X"
 
 
@@ -109,6 +109,12 @@ def alg_bytes(M, N, K, out_type):
 
 def workload_name(M, N, K, out_type):
     return f"mxfp6_gemm_{M}x{N}x{K}_{mx.OUT_NAMES[out_type]}"
+
+
+def tile_kernel_name(w):
+    """The kernel that a Workload's plan spends its time in."""
+    return KERNEL_NAMES[mx.plan_kernel(w.ot, w.M, w.N, w.p.Kp, w.tile, w.S,
+                                       mx.A_REPACK if w.repack else mx.A_ROWS, w.p.a_row_bytes)[0]]
 
 
 def profiled_traffic(workload, kernel):
@@ -392,7 +398,7 @@ def headline(name, steps, warmup, ref, w=None):
     tflops = w.flops / (ms * 1e-3) / 1e12
 
     # dominant kernel: the same launches issued one by one, HIP events around the tile kernel
-    kernel_name = "wide_kernel" if tuple(w.tile) in WIDE_TILES else "slab_kernel"
+    kernel_name = tile_kernel_name(w)
     if w.S == 1 and w.repack:
         ash = torch.empty(mx.preshuffled_bytes(M, p.Kp), dtype=torch.uint8, device="cuda:0")
         evs = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))

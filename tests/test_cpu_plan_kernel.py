@@ -98,3 +98,17 @@ def test_loaded_skinny_plan_reads_rows(mx, tmp_path):
         assert mx.gemm_plan(1, M, N, Kp, 0) == (tuple(tile), 1, False)
     finally:
         mx.tune_reset()
+
+
+@pytest.mark.parametrize("M,N,K,want", [(256, 256, 1024, "tiny_kernel"), (8192, 8192, 8192, "wide_kernel"),
+                                        (2048, 5120, 105728, "wide_kernel"),
+                                        (64, 28672, 8192, "stream_kernel"),
+                                        (256, 18432, 12288, "stream_kernel")])
+def test_bench_names_the_kernel(mx, M, N, K, want):
+    import types
+    import bench
+    Kp = mx.kpad(K)
+    w = types.SimpleNamespace(ot=mx.OUT_F16, M=M, N=N, tile=mx.choose_tile(M, N, Kp),
+                              S=mx.splitk_segments(M, N, Kp), repack=mx.repacks_a(M, N, Kp),
+                              p=types.SimpleNamespace(Kp=Kp, a_row_bytes=mx.packed_bytes(K)))
+    assert bench.tile_kernel_name(w) == want
