@@ -35,7 +35,7 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[MPW][NPW], OutT* __
             // stored together, 128 contiguous bytes of a row (two of them) an instruction. Against a
             // block at a time (four half lines an instruction), three operand sets in turn: 8192 x
             // 8192 x 1024 76.7 -> 71.0 us, 8192 x 8192 x 2048 130 -> 118, 4096 x 4096 x 1024 24.0 ->
-            // 19.3, 8192 x 28672 x 1024 254 -> 220, 8192^3 349 -> 340.
+            // 19.3, 8192 x 28672 x 1024 254 -> 220 (8192^3: within the noise).
             const bool odd = (lane & 1) != 0;
             const uint32_t sel_send = odd ? 0x05040100u : 0x07060302u;
             const uint32_t sel_a = odd ? 0x03020504u : 0x05040100u;

@@ -17,17 +17,21 @@
 //   sync    one workgroup barrier per chunk: the copying wave has waited for chunk g + 1 (its own
 //           vmcnt count: it issues nothing else), every computing wave for its reads of chunk g,
 //           whose buffer then takes chunk g + NB.
-// What bounds it: a CU keeps only about 32 KB of cache misses in flight (its L1's lines), whether
-// they go to registers or to LDS: 64 x 8192 x 8192 on 64 CUs moved 29 KB/us a CU from HBM and 48 from
-// the Infinity Cache, the same with 2, 4 or 6 K-tiles of loads ahead. So lead past two K-tiles is
-// worth nothing; the lines of A, the padded scale dwords and the number of CUs in use are what
-// counts. That is why A comes in two K-tiles per row piece, only one wave loads A's scales, and WN
-// shrinks when the grid is small (tile_dispatch.hpp). 64 x 28672 x 8192 (three operand sets in turn,
-// B from HBM): 52.1 us on the slab kernel (B and A through LDS a slab at a time, every wave
-// copying), 38.2 here: 5.0 TB/s of operands; without A's copies and scales 30.5.
-// NT: B's loads are nontemporal where B exceeds half the last-level cache and is read by one tile
-// row: 44.8 -> 39.1 us at 64 x 28672 x 8192 (B 176 MB), while B that would have stayed in the cache
-// loses (64 x 8192 x 8192, B 50 MB: 20.9 -> 31.4 us).
+// What bounds it: the read requests a CU keeps in flight, about a hundred of at most 128 bytes, whether
+// they go to registers or to LDS (104 a CU on 64 x 28672 x 8192 and 93 on the bands of 256 x 18432 x 12288
+// by the counters, profiles/stream_kernel_*_pmc.txt; MFMAs busy 8 and 18% of the cycles): 64 x 8192 x 8192
+// on 64 CUs moved 29 KB/us a CU from HBM and 48 from the Infinity Cache, the same with 2, 4 or 6 K-tiles
+// of loads ahead. So lead past two K-tiles is worth nothing; the lines of A, the padded scale dwords and
+// the number of CUs in use are what counts. That is why A comes in two K-tiles per row piece, only one wave
+// loads A's scales, and WN shrinks when the grid is small (tile_dispatch.hpp). 64 x 28672 x 8192 (three
+// operand sets in turn, B from HBM): 52.1 us on the slab kernel (B and A through LDS a slab at a time,
+// every wave copying), 38.2 here: 5.0 TB/s of operands; without A's copies and scales 30.5.
+// NT: B's loads are nontemporal where B exceeds half the last-level cache and is read by one tile row. A
+// layer's weights are read again only after the other layers': with three or more sets in turn 24 plans
+// of 140-271 MB of B are 7-15% faster so (64 x 28672 x 8192 43.4 -> 38.0 us, 32 x 28672 x 6400 34.4 ->
+// 30.9), and prepare_b followed by the GEMM 4-7%. The same B again at once loses what the cache would
+// have kept (140-212 MB: 3-26%, 64 x 28672 x 8192 32.4 -> 36.9; 64 x 8192 x 8192, B 50 MB: 20.9 -> 31.4;
+// from 240 MB on 0-8%).
 // BAND (WN = 0 in the template; 128 rows, scale groups of four row blocks): a wave owns 128 rows and
 // one 32-column block, byte blk % npw of its scale group of npw blocks, so that the launch can
 // choose how many columns a workgroup takes (2 to 5 computing waves, all in one round of the CUs)

@@ -84,7 +84,8 @@ int mxfp6_hip_prep_few_waves(int rows, int cols);
 
 /* Quantisation and layout kernels (csrc/hip/prep_kernel.hpp). All return 0 ok, 2 launch error.
  *
- * Row-major float x[rows][cols] (4-byte aligned; 16-byte aligned with cols % 4 == 0 reads float4):
+ * Row-major float x[rows][cols] (4-byte aligned; 16-byte aligned with cols % 4 == 0 reads float4 where
+ * the output is preshuffled):
  * for each row r and block c < nblk, the codes of values 32c .. 32c+31 (zero past cols; zero bytes
  * for a block past the values) go to packed + r * row_bytes + 24c, cut at row_bytes (row_bytes % 4
  * == 0) -- or, with preshuffled != 0, to the preshuffled operand layout at Kp (nblk = Kp / 32,

@@ -56,14 +56,14 @@ inline int stream_waves(const mxfp6_launch_desc& d, long cus, bool nt_b) {
 }
 
 // Computing waves of the 128-row bands that run a wide tile's plan on row-major A, or 0 where the wide
-// kernel is the better one: the fewest with which the plan's workgroups run in one round of the CUs. Up
-// to four were never slower than the wide kernel on 43 measured shapes (three waves 2048 x 1152 x 2128
-// 1.25x, 128 x 24576 x 4096 1.52x; four 512 x 8192 x 2048 1.00x, 1203 x 2560 x 1408 1.12x, 128 x 2048 x
-// 50116 in 16 segments 1.16x); five only where B is no small part of the 256 MiB last-level cache (57
-// MB 1.03-1.08x unsplit, 0.90 split; 75 MB 1.29x, 126 MB in two segments 1.18x, 170 MB 1.32x; 28 MB
-// 0.91, 42 MB 1.00), for there the wide kernel's loads, one K-tile ahead, wait on HBM; six lost but
-// for one shape (682 x 1280 x 27520 in 6 segments 0.76, 256 x 7040 x 9920 in 3 0.89; 128 x 6016 x 18944
-// in 8 1.15x). Segments of fewer than eight K-tiles keep the wide kernel, which has short paths for them.
+// kernel is the better one: the fewest with which the plan's workgroups run in one round of the CUs. On 110
+// routed plans drawn at random the bands were 1.09-1.60x as fast as the wide kernel
+// (profiles/bands_against_wide_tiles.txt: three waves 1.44x on average, four 1.32x, five 1.19x). Five only
+// where B is no small part of the 256 MiB last-level cache (57 MB 1.03-1.08x unsplit, 0.90 split; 75 MB 1.29x,
+// 126 MB in two segments 1.18x, 170 MB 1.32x; 28 MB 0.91, 42 MB 1.00), for there the wide kernel's loads, one
+// K-tile ahead, wait on HBM; six lost but for one shape (682 x 1280 x 27520 in 6 segments 0.76, 256 x 7040 x
+// 9920 in 3 0.89; 128 x 6016 x 18944 in 8 1.15x). Segments of fewer than eight K-tiles keep the wide
+// kernel, which has short paths for them.
 inline int band_waves(const mxfp6_launch_desc& d, long cus) {
     if (d.a_layout != MXFP6_A_ROWS || d.out_stream || d.Kp / 192 < 8 * d.splits) return 0;
     const long rows = ceil_div(d.M, 128) * d.splits, blks = ceil_div(d.N, 32);
