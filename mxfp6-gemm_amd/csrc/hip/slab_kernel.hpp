@@ -431,11 +431,12 @@ int wide_launch_t(const mxfp6_launch_desc* d, const mxfp6_dispatch::TileRun& run
 }
 
 // The skinny tiles: row-major A on the stream kernel, or on 128 x 256 wide tiles that read the skinny
-// tile's scale groups; A repacked or preshuffled on the slab kernel with one wave row and four wave
-// columns. All give the same bits.
+// tile's scale groups; A repacked or preshuffled, and one K-tile of row-major A but for 32 x 256, on the slab
+// kernel with one wave row and four wave columns (tile_dispatch.hpp). All give the same bits.
 template <int MT, int NT, typename KT, bool SPLIT>
 int skinny_launch(const mxfp6_launch_desc* d, const mxfp6_dispatch::TileRun& run, hipStream_t st) {
-    if (run.kernel == MXFP6_TILE_SLAB) return slab_launch_t<MT, NT, 1, 4, 4, 8, KT, SPLIT, false>(d, st);
+    if (run.kernel == MXFP6_TILE_SLAB)
+        return slab_launch_t<MT, NT, 1, 4, 4, 8, KT, SPLIT, MT == 64 || NT == 128>(d, st);
     if (run.kernel == MXFP6_TILE_WIDE) {
         using G = WideGeom<4, 2, WIDE_NB, false, MT / 32, NT / 128>;
         const dim3 grid((unsigned)((d->M + G::MT - 1) / G::MT), (unsigned)((d->N + G::NT - 1) / G::NT),
@@ -463,7 +464,7 @@ int slab_run(const mxfp6_launch_desc* d, hipStream_t st) {
     if (d->MT == 128 && d->NT == 256 && d->mpw == 4) return wide_launch_t<4, 2, 8, KT, SPLIT>(d, run, st);
     if (d->MT == 256 && d->NT == 256 && d->npw == 2) return wide_launch_t<8, 2, 4, KT, SPLIT>(d, run, st);
     if (d->MT == 128 && d->NT == 384) return wide_launch_t<4, 3, 8, KT, SPLIT>(d, run, st);
-    // skinny tiles: the stream kernel on row-major A, here preshuffled A (a deeper ring)
+    // skinny tiles (a deeper ring where this kernel runs them)
     if (d->MT == 32 && d->NT == 128) return skinny_launch<32, 128, KT, SPLIT>(d, run, st);
     if (d->MT == 32 && d->NT == 256) return skinny_launch<32, 256, KT, SPLIT>(d, run, st);
     if (d->MT == 64 && d->NT == 128) return skinny_launch<64, 128, KT, SPLIT>(d, run, st);

@@ -21,6 +21,14 @@ inline double b_bytes(const mxfp6_launch_desc& d) { return (double)d.N * (d.Kp /
 
 constexpr double LLC_HALF = 128.0 * (1 << 20);  // half of MI355X's 256 MiB last-level cache
 
+// The skinny tile's workgroups against the rounds of the CUs that 128 x 256 wide tiles would take: the
+// workgroups a CU of the skinny tile in the time of a round of wide ones.
+inline double skinny_rounds(const mxfp6_launch_desc& d, long cus) {
+    const long tile = ceil_div(d.M, d.MT) * ceil_div(d.N, d.NT) * d.splits;
+    const long wide = ceil_div(d.M, 128) * ceil_div(d.N, 256) * d.splits;
+    return (double)tile / (double)(cus * ceil_div(wide, cus));
+}
+
 // Whether a skinny tile's plan (32 or 64 rows) on row-major A runs on 128 x 256 wide tiles with the
 // skinny tile's scale groups: by the work of the busiest CU. A round of wide workgroups takes as long
 // as 1.1 (64 x 256), 1.4 (32 x 256) or 2 (the 128-column tiles) of the skinny tile's workgroups a CU,
@@ -29,13 +37,23 @@ constexpr double LLC_HALF = 128.0 * (1 << 20);  // half of MI355X's 256 MiB last
 // (539 routed plans) the rule's pick is 1.0% slower than the better of the two on average and 1.37x at
 // worst (448 x 5760 x 16320 in 3 segments, stream 102.8 us, wide 74.9). One tile row never goes wide
 // (32 x 32768 x 1024: stream 9.3 us, wide 15.2; 64 x 32768 x 8192: 41.3 and 64.8), many rows do (2784
-// x 2304 x 11392: stream 142.8, wide 79.9).
+// x 2304 x 11392: stream 142.8, wide 79.9). `one` K-tile a segment, on 32 x 128: from 4.2 (slab 13.2 us,
+// wide 14.1 at 3.97, 608 x 13696; 16.0 and 14.4 at 4.8, 3168 x 3200).
 // Rows whose 128 offsets pass 32 bits stay on the tile's own kernel.
-inline bool skinny_runs_wide(const mxfp6_launch_desc& d, long cus) {
-    const long tile = ceil_div(d.M, d.MT) * ceil_div(d.N, d.NT) * d.splits;
-    const long wide = ceil_div(d.M, 128) * ceil_div(d.N, 256) * d.splits;
-    const long tenths = d.NT == 128 ? 20 : d.MT == 64 ? 11 : 14;
-    return 10 * tile > tenths * cus * ceil_div(wide, cus) && 127.0 * d.A_row_bytes < 2147483648.0;
+inline bool skinny_runs_wide(const mxfp6_launch_desc& d, long cus, bool one) {
+    const double least = d.NT == 256 ? (d.MT == 64 ? 1.1 : 1.4) : one && d.MT == 32 ? 4.2 : 2.0;
+    return skinny_rounds(d, cus) > least && 127.0 * d.A_row_bytes < 2147483648.0;
+}
+
+// Whether a skinny tile's plan of one K-tile a segment that does not go wide runs on the slab kernel: the
+// stream kernel loads two ahead. 64 x 128 (slab 4.1-4.9 us, stream 4.6-5.6 on 10 plans) and 64 x 256 on no more
+// workgroups than CUs (four waves; 5.2-6.6 against 5.5-7.1), on more where no block is masked (10.5 and 11.7 at
+// 832 x 9472; masked 10.4 and 9.3 at 832 x 5248); 32 x 128 on more than two workgroups a CU (7.3 and 8.1 at
+// 1120 x 3712; to two within 5% either way). From two K-tiles on the stream kernel is as fast or
+// faster (profiles/skinny_tiles_short_k.txt).
+inline bool one_k_tile_on_slab(const mxfp6_launch_desc& d, long cus, int waves) {
+    if (d.MT == 64) return d.NT == 128 || waves == 4 || (d.M % 64 == 0 && d.N % 256 == 0);
+    return d.NT == 128 && skinny_rounds(d, cus) > 2.0;
 }
 
 // Computing waves of a stream workgroup (four as the router counts the tile): fewer where four would
@@ -89,9 +107,11 @@ inline TileRun tile_run(const mxfp6_launch_desc& d, long cus) {
         return {MXFP6_TILE_BAND, waves, d.M <= 128 && b_bytes(d) > LLC_HALF};
     }
     if (d.MT > 64 || d.a_layout != MXFP6_A_ROWS) return {MXFP6_TILE_SLAB, 0, false};
-    if (skinny_runs_wide(d, cus)) return {MXFP6_TILE_WIDE, 0, false};
+    const bool one = d.Kp / 192 <= d.splits;  // K-tile a segment
+    if (skinny_runs_wide(d, cus, one)) return {MXFP6_TILE_WIDE, 0, false};
     const bool nt_b = d.M <= d.MT && b_bytes(d) > LLC_HALF;
     const int waves = stream_waves(d, cus, nt_b);
+    if (one && one_k_tile_on_slab(d, cus, waves)) return {MXFP6_TILE_SLAB, 0, false};
     return {MXFP6_TILE_STREAM, waves, nt_b && waves == 4};
 }
 

@@ -7,6 +7,7 @@ import pytest
 
 PROFILE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "profiles",
                        "skinny_tiles_on_row_major_a.txt")
+SHORT = PROFILE.replace("on_row_major_a", "short_k")
 
 
 def _skinny_times():
@@ -32,6 +33,32 @@ def test_skinny_tiles_run_on_the_faster_kernel(mx):
         over.append(us / min(t["stream"], t["wide"]))
         assert over[-1] < 1.4, (M, N, K, MT, NT, S, t)
     assert len(over) > 400 and math.exp(sum(map(math.log, over)) / len(over)) < 1.01
+
+
+def test_short_skinny_plans_run_on_the_faster_kernel(mx):
+    """One to seven K-tiles a segment: none slower than on the slab kernel by more than 8%, 4% for one
+    K-tile (and 0.2 us, the spread of the launches that set the times of about 4 us)."""
+    n = 0
+    with open(SHORT) as f:
+        lines = [line.split() for line in f if not line.startswith("#")]
+    for v in lines:
+        nk, M, N, K, MT, NT, S = map(int, v[:7])
+        us = float(v[{"slab": 7, "stream": 8, "wide": 9}[_kernel(mx, M, N, K, MT, NT, S)[0]]])
+        assert us <= float(v[7]) * (1.04 if nk == 1 else 1.08) + 0.2, v
+        n += 1
+    assert n > 300
+
+
+@pytest.mark.parametrize("MT,NT,want", [(64, 128, "slab"), (64, 256, "slab"), (32, 128, "stream"),
+                                        (32, 256, "stream")])
+def test_one_k_tile(mx, MT, NT, want):
+    assert _kernel(mx, 320, 3584, 130, MT, NT, 1)[0] == want
+    assert _kernel(mx, 96, 3584, 576, MT, NT, 3)[0] == want
+    assert _kernel(mx, 320, 3584, 384, MT, NT, 1)[0] == "stream"
+    assert _kernel(mx, 1120, 3712, 192, 32, 128, 1)[0] == "slab"
+    assert _kernel(mx, 832, 9472, 192, 64, 256, 1)[0] == "slab"
+    assert _kernel(mx, 832, 5248, 192, 64, 256, 1)[0] == "stream"
+    assert _kernel(mx, 4096, 8192, 192, MT, NT, 1)[0] == "wide"
 
 
 @pytest.mark.parametrize("MT,NT", [(32, 128), (32, 256), (64, 128), (64, 256)])

@@ -1,7 +1,8 @@
 """The stream kernel (stream_kernel.hpp): the skinny tiles on row-major A. Bit for bit the output of
 the direct kernel, and on ragged shapes of the slab kernel on the repacked A, where its chunks (two
 K-tiles), its passes, its number of computing waves, its masks, its output type and its loads of B change. Every
-case says how many computing waves it is for, and the plan's kernel is asked."""
+case says how many computing waves it is for, and the plan's kernel is asked. One K-tile a segment runs on the slab
+kernel where that is faster: row-major A there, against the same references."""
 import numpy as np
 import pytest
 import torch
@@ -26,8 +27,9 @@ def problem(M, N, K, seed, **kw):
 
 def streams(dp, out_type, S, waves):
     p = dp.p
-    assert mx.plan_kernel(out_type, p.M, p.N, p.Kp, dp.tile, S,
-                          A_row_bytes=p.a_row_bytes) == ("stream", waves, False)
+    slab = p.Kp // 192 <= S and dp.tile[0] == 64
+    assert mx.plan_kernel(out_type, p.M, p.N, p.Kp, dp.tile, S, A_row_bytes=p.a_row_bytes) == (
+        ("slab", 0, False) if slab else ("stream", waves, False))
 
 
 @pytest.mark.parametrize("K", [192, 384, 576, 768, 960])
@@ -65,8 +67,20 @@ def test_stream_split_bitwise_equals_direct(tile, M, N, waves, K, S):
 def test_stream_ragged_equals_slab(tile, M, N, K, S, compact):
     dp = g.DevProblem(problem(M, N, K // 32 * 32, M + K, compact=compact), tile)
     p = dp.p
-    assert mx.plan_kernel(mx.OUT_F32, M, N, p.Kp, tile, S, A_row_bytes=p.a_row_bytes)[0] == "stream"
+    assert mx.plan_kernel(mx.OUT_F32, M, N, p.Kp, tile, S, A_row_bytes=p.a_row_bytes)[0] == (
+        "slab" if K == 192 and tile[0] == 64 else "stream")
     same(g.run_explicit(dp, mx.OUT_F32, splits=S), g.run_explicit(dp, mx.OUT_F32, splits=S, a_layout=1))
+
+
+@pytest.mark.parametrize("tile,M,N,K,S", [(T64_128, 37, 545, 96, 1), (T64_128, 130, 260, 350, 2),
+                                          (T64_256, 61, 1001, 192, 1), (T64_256, 832, 9472, 160, 1),
+                                          (T32_128, 1119, 3714, 192, 1), (T32_128, 1120, 3712, 64, 1)])
+@pytest.mark.parametrize("out_type", [mx.OUT_F32, mx.OUT_F16, mx.OUT_BF16])
+def test_one_k_tile_on_rows_equals_repacked(tile, M, N, K, S, out_type):
+    dp = g.DevProblem(problem(M, N, K // 32 * 32, M + K), tile)
+    p = dp.p
+    assert mx.plan_kernel(out_type, M, N, p.Kp, tile, S, A_row_bytes=p.a_row_bytes)[0] == "slab"
+    same(g.run_explicit(dp, out_type, splits=S), g.run_explicit(dp, out_type, splits=S, a_layout=1))
 
 
 @pytest.mark.parametrize("tile,M,N,waves", [(T32_128, 33, 130, 1), (T32_128, 250, 2040, 2),
