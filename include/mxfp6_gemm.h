@@ -183,8 +183,8 @@ int mxfp6_gemm_plan(int out_type, int M, int N, int Kp, size_t ws_bytes, int til
 
 /* Whether the routed plan for (out_type, M, N, Kp, A_row_bytes) writes D with nontemporal stores
  * (unsplit plans whose operands fit in MI355X's 256 MiB last-level cache but whose operands and D
- * together do not, or, D of 16 bits, fill over half of it with a D that is no small part;
- * csrc/host/plan.hpp). The answer is for the plan gemm() runs with the preferred workspace
+ * together do not, or, D of 16 bits, fill over half of it with a D that is no small part; only D
+ * whose rows are whole 128-byte lines, csrc/host/plan.hpp). The answer is for D on a 128-byte boundary and for the plan gemm() runs with the preferred workspace
  * (mxfp6_gemm_preferred_workspace_size) and no measured plan registered for the shape; a measured
  * plan or a shorter workspace can run another plan, whose stores are decided the same way from
  * that plan. No counterpart in the reference (its epilogue stores are plain); D's values are the

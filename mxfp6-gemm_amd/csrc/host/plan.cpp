@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <mutex>
 #include <vector>
@@ -415,14 +416,16 @@ bool streams_output(int out_type, int M, int N, int Kp, const TileChoice& tc, in
     // the split-K partials are read back and the reduce writes D; the other tiles' kernel keeps
     // plain stores
     if (S > 1 || !is_wide(tc)) return false;
+    const int value_bytes = out_type == 0 ? 4 : 2;  // FP32 or a 16-bit type
+    if ((long)N * value_bytes % STREAM_LINE_BYTES != 0) return false;
     const double packed = Kp / 4 * 3.0;
     const double in = (double)M * A_row_bytes + (repack ? ((M + 31) / 32 * 32) * packed : 0.0) +
                       (double)N * packed + (double)(M + N) * (Kp / 32);
-    const double out = (double)M * N * (out_type == 0 ? 4 : 2);  // FP32 or a 16-bit type
+    const double out = (double)M * N * value_bytes;
     if (in > LLC_BYTES) return false;
-    return in + out > STREAM_FOOTPRINT_BYTES ||
-           (out_type != 0 && in + out > LLC_BYTES / 2 &&
-            out >= (in + out <= STREAM_MID_BYTES ? STREAM_MID_RATIO : STREAM_D_RATIO) * in);
+    if (in + out > STREAM_FOOTPRINT_BYTES) return true;
+    if (out_type == 0 || tc.NPW % 2 != 0 || in + out <= LLC_BYTES / 2) return false;
+    return out >= (in + out <= STREAM_MID_BYTES ? STREAM_MID_RATIO : STREAM_D_RATIO) * in;
 }
 
 // The launch descriptor of a plan, without its pointers.
@@ -460,6 +463,7 @@ int run(int out_type, int M, int N, int Kp, const TileChoice& tc, int S, int a_l
     d.sA = dsA;
     d.sB = dsB;
     d.D = dD;
+    if (reinterpret_cast<uintptr_t>(dD) % STREAM_LINE_BYTES != 0) d.out_stream = 0;
     d.ws = S > 1 ? static_cast<float*>(ws) : nullptr;
     d.Ash = a_layout == MXFP6_A_REPACK
                 ? static_cast<uint8_t*>(ws) + (split_bytes(M, N, S) + 255) / 256 * 256

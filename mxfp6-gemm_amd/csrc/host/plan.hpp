@@ -45,10 +45,18 @@ constexpr double PLAN_MIN_GAIN = 0.01;     // lead a more complex plan needs ove
 //   a kernel that reads and writes (8192^3 346.2 -> 329.6 and 388.3 -> 380.2; only reading, 370.7 -> 378.3);
 //   plain stores have stayed there but for D of at least STREAM_D_RATIO times in (short K: 8192x14336x512
 //   96.5 -> 84.9).
+// D whose rows are no whole number of cache lines, or that does not begin on one, is never streamed: a store past
+// the caches writes a part of a line, and the memory has to merge it. Streamed against plain
+// (profiles/gemm_d_stores_by_row_alignment.txt, 280 shapes), odd N: 1.05-2.96 times as long below 280 MB
+// (2091 x 23035 x 2218 159.7 us against 119.6) and 1.00-2.86 above; even N 0.80-2.46 and 0.77-2.49, 1.2 and
+// 1.3 on average; whole lines 0.91. Tiles of an odd number of blocks a wave (128x384) store the last one's
+// rows as half lines: below 280 MB 0.90-1.02 alone on average and 1.04-1.09 with a reader that writes, so not
+// there.
 // FP32 D up to STREAM_FOOTPRINT_BYTES is stored the ordinary way: what reads it next is prepare_a, and the pair
 // is 3-8% slower with D streamed (4096x8192x2048 96.7 -> 105.5 us, one D 85.6 -> 100.1), as the GEMM alone
 // is where D is one buffer (60.2 -> 71.1).
 constexpr double LLC_BYTES = 268435456.0;
+constexpr long STREAM_LINE_BYTES = 128;
 constexpr double STREAM_FOOTPRINT_BYTES = 280e6;
 constexpr double STREAM_MID_BYTES = 236e6;
 constexpr double STREAM_MID_RATIO = 0.4;

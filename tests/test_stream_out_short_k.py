@@ -1,6 +1,6 @@
 """Unsplit plans on wide tiles whose operands and 16-bit D fill half the 256 MiB last-level cache or more
 write D with nontemporal stores where D is at least 0.4 times the operands (up to 236 MB in all) or 8 times
-(above), FP32 D only past 280 MB: the rule's edges, and the values against the direct kernel bit for bit."""
+(above), FP32 D only past 280 MB, and either only in rows of whole 128-byte lines: the rule's edges, and the values against the direct kernel bit for bit."""
 import pytest
 
 import checks
@@ -21,10 +21,17 @@ import mxfp6_amd as mx
     (4096, 16384, 512, mx.OUT_F32, False),    # 268 + 8 MB
     (4096, 17408, 512, mx.OUT_F32, True),     # 285 + 8 MB
     (4096, 10240, 1024, mx.OUT_F16, False),
-    (2048, 28672, 1024, mx.OUT_F16, True)])
+    (2048, 28672, 1024, mx.OUT_F16, True),
+    # rows that are no whole number of 128-byte lines, below and above 280 MB
+    (2091, 23035, 2218, mx.OUT_BF16, False), (8192, 8194, 1024, mx.OUT_BF16, False),
+    (8191, 8224, 1024, mx.OUT_F16, False), (8191, 8256, 1024, mx.OUT_F16, True),
+    (2048, 102271, 1024, mx.OUT_F16, False), (2048, 102272, 1024, mx.OUT_F16, True),
+    (4096, 17424, 512, mx.OUT_F32, False), (4096, 17472, 512, mx.OUT_F32, True),
+    (10368, 9600, 142, mx.OUT_F16, False)])   # 128x384: three blocks a wave
 def test_rule(M, N, K, out_type, want):
     Kp = mx.kpad(K)
     assert mx.splitk_segments(M, N, Kp) == 1
+    assert mx.plan_kernel(out_type, M, N, Kp, mx.choose_tile(M, N, Kp))[0] in ("wide", "band")
     assert mx.streams_output(out_type, M, N, Kp, mx.packed_bytes(Kp)) == want
 
 
