@@ -30,12 +30,14 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[MPW][NPW], OutT* __
             // that the even lane holds rows +0 and +2 of both columns and the odd lane rows +1
             // and +3 (one quad_perm DPP move and three byte permutes per 4 values), halving the
             // store instructions. The conversions are the per-element ones of cvt_out.
-            // A row of one block is 64 bytes, half a cache line, and D at these widths is bound by
-            // how many lines the stores touch: where a wave owns two blocks side by side they are
-            // stored together, 128 contiguous bytes of a row (two of them) an instruction. Against a
-            // block at a time (four half lines an instruction), three operand sets in turn: 8192 x
-            // 8192 x 1024 76.7 -> 71.0 us, 8192 x 8192 x 2048 130 -> 118, 4096 x 4096 x 1024 24.0 ->
-            // 19.3, 8192 x 28672 x 1024 254 -> 220 (8192^3: within the noise).
+            // NT: a row of one block is 64 bytes, half a cache line, which the memory takes badly past the
+            // caches. Where a wave owns two blocks side by side they are stored together, 128
+            // contiguous bytes of a row (two of them) an instruction: against a block at a time (four half
+            // lines an instruction) 8192 x 8192 x 1024 76.7 -> 71.0 us, 8192 x 28672 x 1024 254 -> 220. Stores
+            // through the caches merge there, and the second trade costs up to 3% (529 plans, 1% on
+            // average, profiles/epilogue16_plain_stores.txt: 8192 x 6144 x 512 40.3 us against 39.3, 3000 x 5000 x
+            // 4096 46.1 and 45.8; only with N a power of two it gained, 8192^3 348 and 352).
+            constexpr int PAIRED = NT ? NPW / 2 * 2 : 0;
             const bool odd = (lane & 1) != 0;
             const uint32_t sel_send = odd ? 0x05040100u : 0x07060302u;
             const uint32_t sel_a = odd ? 0x03020504u : 0x05040100u;
@@ -61,7 +63,7 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[MPW][NPW], OutT* __
 #pragma unroll
             for (int mi = 0; mi < MPW; mi++) {
 #pragma unroll
-                for (int ni = 0; ni + 1 < NPW; ni += 2)
+                for (int ni = 0; ni + 1 < PAIRED; ni += 2)
 #pragma unroll
                     for (int g = 0; g < 4; g++) {
                         // the pair trades again: the even lane holds all four rows of block ni, the
@@ -77,17 +79,17 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[MPW][NPW], OutT* __
                         put(m + 2, n, odd ? rb : b0);
                         put(m + 3, n, odd ? b1 : rb);
                     }
-                if constexpr (NPW % 2 != 0) {
+#pragma unroll
+                for (int ni = PAIRED; ni < NPW; ni++)
 #pragma unroll
                     for (int g = 0; g < 4; g++) {
                         uint32_t oa, ob;
-                        rows4(acc[mi][NPW - 1], g, oa, ob);
-                        const int m = m_p + mi * 32 + 8 * g, n = n_p + (NPW - 1) * 32;
+                        rows4(acc[mi][ni], g, oa, ob);
+                        const int m = m_p + mi * 32 + 8 * g, n = n_p + ni * 32;
                         if (MASK && n >= N) continue;
                         put(m, n, oa);
                         put(m + 2, n, ob);
                     }
-                }
             }
             return;
         }

@@ -1,6 +1,6 @@
-"""The 16-bit epilogue (epilogue.hpp) stores two 32-column blocks of a wave together, full cache lines of
-a row, and a last odd block by itself: each value is the tile's FP32 result rounded once, at every
-column remainder of a pair of blocks, with nothing written outside D."""
+"""The 16-bit epilogue (epilogue.hpp): each value is the tile's FP32 result rounded once, at every column
+remainder of a pair of blocks, with nothing written outside D. (Streamed D, which is stored two blocks of a wave
+together, is in test_stream_out_short_k.py.)"""
 import numpy as np
 import pytest
 import torch

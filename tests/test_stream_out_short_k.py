@@ -45,3 +45,27 @@ def test_equals_direct_kernel(M, N, K, out_type):
     assert mx.streams_output(out_type, M, N, p.Kp, p.a_row_bytes)
     dp = DevProblem(p, mx.choose_tile(M, N, p.Kp))
     assert (run_routed(dp, out_type).view("u4") == run_direct(dp, out_type).view("u4")).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(2040, 28736, 1344),    # 256 x 256 or 128 x 512 tiles, masked on both sides
+                                   (8191, 8256, 1024), (8100, 8384, 320), (16000, 4672, 384)])
+@pytest.mark.parametrize("out_type,name", [(mx.OUT_F16, "float16"), (mx.OUT_BF16, "bfloat16")])
+def test_masked_in_bounds(M, N, K, out_type, name):
+    """Streamed D of tiles that divide neither M nor N: the FP32 result rounded once, nothing outside."""
+    import torch
+    from gpu_util import DevProblem, run_explicit
+    guard, dtype = 4096, getattr(torch, name)
+    p = checks.spread_scales(mx.make_problem(M, N, K, seed=M + N + K), span=3, seed=K)
+    tile = mx.choose_tile(M, N, p.Kp)
+    assert M % tile[0] != 0 and N % tile[1] != 0
+    assert mx.streams_output(out_type, M, N, p.Kp, p.a_row_bytes)
+    dp = DevProblem(p, tile)
+    want = torch.from_numpy(run_explicit(dp, mx.OUT_F32)).reshape(M, N).to(dtype)
+    buf = torch.full((2 * M * N + 2 * guard,), 0x5A, dtype=torch.uint8, device="cuda")
+    rc = mx.gemm_explicit(out_type, M, N, p.Kp, tile, 1, *dp.ptrs(), buf.data_ptr() + guard, p.a_row_bytes)
+    assert rc == 0, mx.STATUS.get(rc, rc)
+    torch.cuda.synchronize()
+    out = buf.cpu()
+    assert torch.equal(out[guard:-guard].view(torch.int16).reshape(M, N), want.view(torch.int16))
+    assert bool((out[:guard] == 0x5A).all()) and bool((out[-guard:] == 0x5A).all())
