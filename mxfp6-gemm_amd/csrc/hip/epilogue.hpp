@@ -2,7 +2,7 @@
 // FP16 or BF16, row-major, ld = N) or, for a split-K segment, to its FP32 partials ws[z][M][N].
 // Lane l of block (mi, ni) holds column n_w + 32 ni and rows m_w + 32 mi + 8 g + r in
 // acc[mi][ni][4 g + r], with m_w = (first row of the wave) + 4 (l / 32) and n_w = (first column of
-// the wave) + l % 32. MASK stores only rows < M and columns < N. NT writes D with nontemporal
+// the wave) + l % 32. PAIR stores two side-by-side blocks of 16-bit D together. MASK stores only rows < M and columns < N. NT writes D with nontemporal
 // stores (streamed past the caches, for plans whose D would evict the operands the tiles re-read).
 #pragma once
 #include "device_common.hpp"
@@ -20,7 +20,7 @@ __device__ __forceinline__ void store_out(T* p, T v) {
         __builtin_nontemporal_store(v, p);
 }
 
-template <int MPW, int NPW, typename OutT, bool SPLIT, bool MASK, bool NT = false>
+template <int MPW, int NPW, typename OutT, bool SPLIT, bool MASK, bool NT = false, bool PAIR = NT>
 __device__ __forceinline__ void store_tile(const v16f (&acc)[MPW][NPW], OutT* __restrict__ D,
                                            float* __restrict__ ws, int M, int N, int m_w, int n_w,
                                            int lane, int wg_z) {
@@ -30,14 +30,14 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[MPW][NPW], OutT* __
             // that the even lane holds rows +0 and +2 of both columns and the odd lane rows +1
             // and +3 (one quad_perm DPP move and three byte permutes per 4 values), halving the
             // store instructions. The conversions are the per-element ones of cvt_out.
-            // NT: a row of one block is 64 bytes, half a cache line, which the memory takes badly past the
-            // caches. Where a wave owns two blocks side by side they are stored together, 128
-            // contiguous bytes of a row (two of them) an instruction: against a block at a time (four half
-            // lines an instruction) 8192 x 8192 x 1024 76.7 -> 71.0 us, 8192 x 28672 x 1024 254 -> 220. Stores
-            // through the caches merge there, and the second trade costs up to 3% (529 plans, 1% on
-            // average, profiles/epilogue16_plain_stores.txt: 8192 x 6144 x 512 40.3 us against 39.3, 3000 x 5000 x
-            // 4096 46.1 and 45.8; only with N a power of two it gained, 8192^3 348 and 352).
-            constexpr int PAIRED = NT ? NPW / 2 * 2 : 0;
+            // PAIR: a row of one block is 64 bytes, half a cache line. Where a wave owns two blocks side by
+            // side they are stored together, 128 contiguous bytes of a row (two of them) an instruction
+            // in place of four half lines. Past the caches (NT) half lines are slow: 8192 x 8192 x 1024
+            // 76.7 -> 71.0 us with pairs, 8192 x 28672 x 1024 254 -> 220. Stores through the caches merge there,
+            // and the second trade costs up to 3% (profiles/epilogue16_plain_stores.txt: 8192 x 6144 x 512
+            // 39.3 -> 40.3, 3000 x 5000 x 4096 45.8 -> 46.1), but for whole 256 x 256 tiles of long K
+            // (wide_launch_st).
+            constexpr int PAIRED = PAIR ? NPW / 2 * 2 : 0;
             const bool odd = (lane & 1) != 0;
             const uint32_t sel_send = odd ? 0x05040100u : 0x07060302u;
             const uint32_t sel_a = odd ? 0x03020504u : 0x05040100u;

@@ -393,12 +393,25 @@ int slab_launch_t(const mxfp6_launch_desc* d, hipStream_t st) {
 // noise on 8192^3, 2048x1024x105728 and 2048x6144x16128 for 128 x 512), 4 for 256 x 256.
 constexpr int WIDE_NB = 3;
 // an unsplit plan may write D with nontemporal stores (d->out_stream): its own instantiation, so
-// that the kernels with plain stores keep a single epilogue
+// that the kernels with plain stores keep a single epilogue. Of those, whole 256 x 256 tiles of row-major A
+// and K from 4096 on store 16-bit D in pairs of blocks as well (46 plans 0.978-1.007 of the time without,
+// 8192^3 353 -> 347 us; shorter K 1.003-1.02, the other tiles 1.00-1.02: profiles/epilogue16_plain_stores.txt).
+constexpr int PAIR_KP = 4096;
 template <int MB, int NPW, int XG, typename KT, bool SPLIT, bool ASH, bool MASK>
 hipError_t wide_launch_st(const mxfp6_launch_desc* d, const uint8_t* A, hipStream_t st) {
     if constexpr (!SPLIT) {
         if (d->out_stream)
             return wide_kernel_launch<MB, NPW, WIDE_NB, XG, KT, SPLIT, ASH, MASK, true>(d, A, st);
+    }
+    if constexpr (!SPLIT && !ASH && !MASK && MB == 8 && sizeof(KT) == 2) {
+        using G = WideGeom<MB, NPW, WIDE_NB>;
+        if (d->a_layout == MXFP6_A_ROWS && d->Kp >= PAIR_KP)
+            return launch_kernel(wide_kernel<MB, NPW, WIDE_NB, XG, KT, false, false, false, false, 0, false,
+                                             4, NPW, true>,
+                                 dim3((unsigned)(d->M / G::MT), (unsigned)(d->N / G::NT)),
+                                 dim3(G::THREADS), st, A, static_cast<const uint8_t*>(d->Bsh), d->sA,
+                                 d->sB, static_cast<KT*>(d->D), nullptr, d->M, d->N, d->Kp,
+                                 d->A_row_bytes, 1);
     }
     return wide_kernel_launch<MB, NPW, WIDE_NB, XG, KT, SPLIT, ASH, MASK, false>(d, A, st);
 }

@@ -151,7 +151,7 @@ __device__ __forceinline__ void wide_mfma(v16f (&acc)[MB][NPW], int mi, int ni, 
 }
 
 template <int MB_, int NPW_, int NB_, int XG, typename OutT, bool SPLIT, bool ASH, bool MASK,
-          bool STREAM, int ONE = 0, bool SWZ = false, int GA_ = 4, int GB_ = NPW_>
+          bool STREAM, int ONE = 0, bool SWZ = false, int GA_ = 4, int GB_ = NPW_, bool PAIR = STREAM>
 __global__ void __launch_bounds__(256, 1)
     wide_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ Bsh,
                 const uint8_t* __restrict__ sA, const uint8_t* __restrict__ sB,
@@ -412,7 +412,7 @@ __global__ void __launch_bounds__(256, 1)
             if constexpr (NK >= 2) step(std::integral_constant<int, 1>{});
             if constexpr (NK == 3) step(std::integral_constant<int, 2>{});
             const int le = lane_id();  // recomputed: no lane value stays live across the K loop
-            store_tile<MB, NPW, OutT, SPLIT, MASK, STREAM>(acc, D, ws, M, N,
+            store_tile<MB, NPW, OutT, SPLIT, MASK, STREAM, PAIR>(acc, D, ws, M, N,
                                                         wg_m * MT + 4 * (le >> 5),
                                                         wg_n * NT + wave * NPW * 32 + (le & 31),
                                                         le, wg_z);
@@ -545,7 +545,7 @@ __global__ void __launch_bounds__(256, 1)
     // with nontemporal stores
     wait_vmcnt0();
     const int le = lane_id();  // recomputed: no lane value stays live across the K loop
-    store_tile<MB, NPW, OutT, SPLIT, MASK, STREAM>(acc, D, ws, M, N, wg_m * MT + 4 * (le >> 5),
+    store_tile<MB, NPW, OutT, SPLIT, MASK, STREAM, PAIR>(acc, D, ws, M, N, wg_m * MT + 4 * (le >> 5),
                                                 wg_n * NT + wave * NPW * 32 + (le & 31), le,
                                                 wg_z);
 }

@@ -21,7 +21,19 @@ TILES = [(32, 256, 1, 2), (64, 128, 2, 1), (128, 256, 4, 2), (128, 384, 4, 3), (
                                  (130, 126), (37, 130), (261, 610), (261, 1000), (131, 545)])
 @pytest.mark.parametrize("out_type,dtype", [(mx.OUT_F16, torch.float16), (mx.OUT_BF16, torch.bfloat16)])
 def test_rounded_once_and_in_bounds(tile, M, N, out_type, dtype):
-    p = checks.spread_scales(mx.make_problem(M, N, 320, seed=M + N), span=3, seed=N)
+    rounded_once(tile, M, N, 320, out_type, dtype)
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 256, 4096), (4096, 4352, 4096), (4096, 4352, 4032)])
+@pytest.mark.parametrize("out_type,dtype", [(mx.OUT_F16, torch.float16), (mx.OUT_BF16, torch.bfloat16)])
+def test_long_k_whole_tiles(M, N, K, out_type, dtype):
+    """K on both sides of the line from which whole 256 x 256 tiles store pairs of blocks (more tiles than CUs:
+    they do not run as bands)."""
+    rounded_once((256, 256, 4, 2), M, N, K, out_type, dtype)
+
+
+def rounded_once(tile, M, N, K, out_type, dtype):
+    p = checks.spread_scales(mx.make_problem(M, N, K, seed=M + N), span=3, seed=N)
     dp = g.DevProblem(p, tile)
     want = torch.from_numpy(g.run_explicit(dp, mx.OUT_F32)).reshape(M, N).to(dtype)
     buf = torch.full((2 * M * N + 2 * GUARD,), 0x5A, dtype=torch.uint8, device="cuda")
